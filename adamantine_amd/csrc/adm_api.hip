@@ -369,6 +369,12 @@ void Context::build_merged_tables() {
     }
     mb.maxc = maxc;
   }
+  // one candidate count for the wavefront's look-ups, whatever the materials
+  // of its cells (a candidate past a bin's own breakpoints never counts)
+  double maxc = 1.0;
+  for (int mid = 0; mid < mc.n_materials; ++mid)
+    maxc = std::max(maxc, mc.bins[mid].maxc);
+  for (int mid = 0; mid < mc.n_materials; ++mid) mc.bins[mid].maxc = maxc;
 }
 
 int Context::property_kind() const {
@@ -479,6 +485,13 @@ Context::Context(const adm_problem_desc &d) {
       kc.S[q][i] = lagrange(n1, xs, i, kc.xq[q]);
       kc.Dc[q][i] = lagrange_deriv(n1, kc.xq, i, kc.xq[q]);
     }
+  // a symmetric rule has symmetric weights (to the last bit here; the plane
+  // kernel relies on it)
+  for (int q = 0; q < n1; ++q)
+    if (wq[q] != wq[n1 - 1 - q]) {
+      use_plane = false;
+      plane_tables_ok = false;
+    }
   for (int q = 0; q < n1; ++q)
     for (int i = 0; i < n1; ++i) {
       long double acc = 0.0L;
@@ -499,6 +512,13 @@ Context::Context(const adm_problem_desc &d) {
     if (!sym) {
       use_plane = false;
       plane_tables_ok = false;
+    } else {
+      // Dc S inherits Dc's antisymmetry, and its rows differentiate a
+      // constant to zero; its last bits are made to
+      kc.DcS[0][1] = -(kc.DcS[0][0] + kc.DcS[0][2]);
+      kc.DcS[1][1] = 0.0;
+      kc.DcS[1][2] = -kc.DcS[1][0];
+      for (int i = 0; i < 3; ++i) kc.DcS[2][i] = -kc.DcS[0][2 - i];
     }
   }
   det = 1.0;

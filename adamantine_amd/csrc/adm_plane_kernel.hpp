@@ -5,7 +5,7 @@
 // cell's nodes and, after the z contraction, the x-y plane of quadrature
 // points z = s. The x and y contractions run on the lane's (p+1)^2 values in
 // registers; only the z direction crosses lanes, through a wave-private LDS
-// buffer: one exchange for the evaluation and two for the integration
+// buffer: one exchange for the evaluation and one for the integration
 // (against six in the line-per-lane kernel). A wavefront takes a patch of
 // PX x PY cells of one cell layer (7 x 3 for Q2: 63 lanes; 8 x 4 for Q1:
 // 64 lanes), so the nodes its cells share along x and y are summed inside
@@ -29,12 +29,29 @@
 // by rounding only (1/(rho c_p) comes from the hardware reciprocal refined
 // by two Newton steps).
 //
-// Wave-uniform fast path: when no cell of the wavefront holds powder and no
-// point is at or above the solidus, every point is fully solid, and the
-// mixtures reduce to the solid value (the reference adds the other states
-// with a zero ratio, which changes no bit), without the mushy-zone division.
-// Merged tables find a point's interval with one bin lookup (MergedBins).
-// The heat sources run in a second pass over the cells a beam can reach.
+// What bounds it: latency, not arithmetic or memory. A patch of the
+// 128x64x32 Q2 workload issues for some 2,500 cycles of its wavefront; with
+// the two wavefronts per SIMD that the registers allow, the chains of LDS
+// reads (interval, breakpoint, coefficients), of a patch's global loads and
+// of spilled registers' reloads are what it waits for. Hence:
+//  - one-interval form: a wavefront whose planes are cold and lie in one
+//    table interval each reads the coefficients once per plane and then runs
+//    a point loop without branches or LDS reads (see there);
+//  - the next patch's loads are issued a patch ahead;
+//  - a row's interval look-ups advance together;
+//  - the heat source sits behind a call and scalar constants that follow
+//    from symmetry are not held twice, so that nothing spills: one spilled
+//    register's reload waits for the loads in flight before it;
+//  - the two parts of the integration share one exchange.
+// 128x64x32 Q2, per application (plane + gather + face kernels): 100.4 us
+// before, 77.7 us with these; 64 members of 64x32x16, per RK4 step: 3.17 ms
+// before, 2.32 ms.
+// Wavefronts that are solid across several intervals (one material, no
+// powder, below the solidus) take a path of their own: the mixtures reduce
+// to the solid value (the reference adds the other states with a zero ratio,
+// which changes no bit), without the mushy-zone division. The rest update
+// the phase state point by point. The heat sources run in a second pass over
+// the cells a beam can reach.
 #pragma once
 
 #include "adm_kernels.hpp"
@@ -50,11 +67,15 @@ struct PlaneLanes {
   static constexpr int PY = P == 1 ? 4 : 3;
   static constexpr int cells_per_wave = PX * PY;
   // exchange slot per lane (doubles), even so that slots stay 16-byte
-  // aligned for 128-bit LDS accesses
+  // aligned for 128-bit LDS accesses; a cell's N slots are followed by a
+  // gap that spreads the cells of a 128-bit read over the banks
   static constexpr int slot = (NP + 1) & ~1;
+  static constexpr int cell_slots = N * slot + (P == 1 ? 2 : 0);
   // slots of every lane's cell, including the partial cell of the lanes
   // past the last whole one (Q2: lane 63 addresses cell 21's planes)
-  static constexpr int wave_lds = ((64 + N - 1) / N) * N * slot;
+  static constexpr int exchange = ((64 + N - 1) / N) * cell_slots;
+  // two buffers: the two parts of the integration are exchanged at once
+  static constexpr int wave_lds = 2 * exchange;
   // nodes of a patch: (P PX + 1) x (P PY + 1) per plane, N planes; the
   // patch buffer holds one double per node, [plane][y][x]
   static constexpr int patch_nx = P * PX + 1, patch_ny = P * PY + 1;
@@ -73,29 +94,43 @@ constexpr int kPlaneMergedLds =
     kMergedLds + (int)(sizeof(MergedBins) / sizeof(double));
 static_assert(sizeof(MergedBins) % sizeof(double) == 0, "bins layout");
 
-// Patch coordinates of patch index r of a plane launch, npx x npy patches
-// per cell layer and nz layers: x fastest, then y, then the cell layer; or
-// (ymajor) x fastest, then the cell layer, then y -- the order in which the
-// XCD-aware launch hands each XCD one contiguous range, so that every XCD
-// takes a slab of patch rows through all the layers and as many of the
-// slow layers (powder, melt) as the others.
-struct PlanePatch {
-  int px, py, pz;
-};
-__device__ __forceinline__ PlanePatch plane_patch(int npx, int npy, int nz,
-                                                  bool ymajor, int r) {
-  PlanePatch pp;
-  pp.px = r % npx;
-  const int t = r / npx;
-  if (ymajor) {
-    pp.pz = t % nz;
-    pp.py = t / nz;
-  } else {
-    pp.py = t % npy;
-    pp.pz = t / npy;
+// Patch coordinates of a wavefront's patch index r in a plane launch of
+// npx x npy patches per cell layer and nz layers: x fastest, then y, then
+// the cell layer; or (ymajor) x fastest, then the cell layer, then y -- the
+// order in which the XCD-aware launch hands each XCD one contiguous range,
+// so that every XCD takes a slab of patch rows through all the layers and as
+// many of the slow layers (powder, melt) as the others. The wavefront's next
+// patch is a fixed stride on: the stride is divided once and the coordinates
+// then advance by additions and carries.
+struct PatchWalk {
+  int px, mid, top;        // coordinates: x, then the middle and slow ones
+  int dx, dm, dt;          // the stride's
+  int npx, nmid;
+  __device__ __forceinline__ void start(int npx_, int nmid_, int r,
+                                        int stride) {
+    npx = npx_;
+    nmid = nmid_;
+    px = r % npx;
+    mid = (r / npx) % nmid;
+    top = r / npx / nmid;
+    dx = stride % npx;
+    dm = (stride / npx) % nmid;
+    dt = stride / npx / nmid;
   }
-  return pp;
-}
+  __device__ __forceinline__ void advance() {
+    px += dx;
+    mid += dm;
+    top += dt;
+    if (px >= npx) {
+      px -= npx;
+      ++mid;
+    }
+    if (mid >= nmid) {
+      mid -= nmid;
+      ++top;
+    }
+  }
+};
 
 // 1/x from the hardware reciprocal and two Newton steps (within an ulp or
 // two of the correctly rounded quotient)
@@ -107,21 +142,47 @@ __device__ __forceinline__ double recip(double x) {
   return __builtin_fma(r, e, r);
 }
 
-// Interval j = #{B_k <= T} of a merged table by its bins (MergedBins).
+// Intervals j = #{B_k <= T} of M points in a merged table by its bins
+// (MergedBins). The M look-ups advance together, so that their LDS reads
+// overlap. Two candidates are compared without a branch (B is padded with
+// +inf, and a candidate past a bin's own breakpoints lies above T); tables
+// with more breakpoints in one bin take the loop.
+template <int M>
+__device__ __forceinline__ void merged_bin_intervals(const double *B,
+                                                     const MergedBins &mb,
+                                                     const double (&T)[M],
+                                                     int (&j)[M]) {
+  int k0[M];
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    const double x = (T[i] - mb.lo) * mb.inv_w;
+    int b = (int)x;  // NaN and T below lo give bin 0 after the clamp
+    b = x < 0.0 ? 0 : (b > kMergedBins - 1 ? kMergedBins - 1 : b);
+    k0[i] = mb.k0[b];
+  }
+  const int maxc = __builtin_amdgcn_readfirstlane((int)mb.maxc);
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    const int k1 = k0[i] + 1 < kMergedMax - 1 ? k0[i] + 1 : kMergedMax - 1;
+    j[i] = k0[i] + (B[k0[i]] <= T[i] ? 1 : 0);
+    j[i] += B[k1] <= T[i] ? 1 : 0;
+  }
+  for (int c = 2; c < maxc; ++c)
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      const int k = k0[i] + c < kMergedMax - 1 ? k0[i] + c : kMergedMax - 1;
+      j[i] += B[k] <= T[i] ? 1 : 0;
+    }
+}
+
+// One point's interval.
 __device__ __forceinline__ int merged_bin_interval(const double *B,
                                                    const MergedBins &mb,
                                                    double T) {
-  const double x = (T - mb.lo) * mb.inv_w;
-  int b = (int)x;  // NaN and T below lo give bin 0 after the clamp
-  b = x < 0.0 ? 0 : (b > kMergedBins - 1 ? kMergedBins - 1 : b);
-  const int k0 = mb.k0[b];
-  int j = k0;
-  const int maxc = (int)mb.maxc;
-  for (int c = 0; c < maxc; ++c) {
-    const int k = k0 + c < kMergedMax - 1 ? k0 + c : kMergedMax - 1;
-    j += B[k] <= T ? 1 : 0;
-  }
-  return j;
+  const double t[1] = {T};
+  int j[1];
+  merged_bin_intervals<1>(B, mb, t, j);
+  return j[0];
 }
 
 // A uniform value pinned in scalar registers: loads from constant memory
@@ -133,6 +194,42 @@ template <class T>
 __device__ __forceinline__ T in_sgpr(T x) {
   asm volatile("" : "+s"(x));
   return x;
+}
+
+// Heat-source values of one lane's point plane: slot[q], 1/(rho c_p) of the
+// point on entry, becomes source * 1/(rho c_p) * JxW. Not inlined: few
+// wavefronts come here, and the exponential's constants would otherwise be
+// kept in registers through the whole patch loop (28 registers that it then
+// spills).
+#define ADM_LDS __attribute__((address_space(3)))
+template <int P>
+static __device__ __attribute__((noinline)) void plane_source(
+    ADM_LDS double *slot, const ADM_LDS adm_beam_state *beams, int n_beams,
+    const ADM_LDS CellConstLds *sk, const ADM_CONSTANT KConst *kc, int cx,
+    int cy, int cz, int s) {
+  constexpr int N = P + 1;
+  const double pz = kc->origin[2] + (cz + sk->xq[s]) * kc->h[2];
+  const double det = kc->det, wz = sk->wq[s];
+#pragma unroll 1
+  for (int qy = 0; qy < N; ++qy) {
+    const double py = kc->origin[1] + (cy + sk->xq[qy]) * kc->h[1];
+    double qs[N];
+#pragma unroll
+    for (int qx = 0; qx < N; ++qx) qs[qx] = 0.0;
+#pragma unroll 1
+    for (int b = 0; b < n_beams; ++b)
+#pragma unroll
+      for (int qx = 0; qx < N; ++qx) {
+        const double px = kc->origin[0] + (cx + sk->xq[qx]) * kc->h[0];
+        qs[qx] += beam_value(*(const adm_beam_state *)(beams + b), px, py, pz,
+                             kc->log_01);
+      }
+#pragma unroll
+    for (int qx = 0; qx < N; ++qx) {
+      const double jxw = det * ((sk->wq[qx] * sk->wq[qy]) * wz);
+      slot[qx + N * qy] = (qs[qx] * slot[qx + N * qy]) * jxw;
+    }
+  }
 }
 
 // wavefronts per SIMD the plane kernel is compiled for (VGPR budget)
@@ -263,10 +360,17 @@ __global__ void __launch_bounds__(256)
     Dc[2][0] = -d02;
     Dc[2][1] = -d01;
     Dc[2][2] = -d00;
-#pragma unroll
-    for (int q = 0; q < N; ++q)
-#pragma unroll
-      for (int k = 0; k < N; ++k) DS[q][k] = in_sgpr(kc.DcS[q][k]);
+    const double e00 = in_sgpr(kc.DcS[0][0]), e01 = in_sgpr(kc.DcS[0][1]),
+                 e02 = in_sgpr(kc.DcS[0][2]), e10 = in_sgpr(kc.DcS[1][0]);
+    DS[0][0] = e00;
+    DS[0][1] = e01;
+    DS[0][2] = e02;
+    DS[1][0] = e10;
+    DS[1][1] = 0.0;
+    DS[1][2] = -e10;
+    DS[2][0] = -e02;
+    DS[2][1] = -e01;
+    DS[2][2] = -e00;
   } else {
 #pragma unroll
     for (int q = 0; q < N; ++q)
@@ -277,12 +381,9 @@ __global__ void __launch_bounds__(256)
         DS[q][k] = in_sgpr(kc.DcS[q][k]);
       }
   }
-  const double ih0 = in_sgpr(kc.inv_h[0]), ih1 = in_sgpr(kc.inv_h[1]),
-               ih2 = in_sgpr(kc.inv_h[2]);
-  const double det = in_sgpr(kc.det);
-  double wq[N];
-#pragma unroll
-  for (int q = 0; q < N; ++q) wq[q] = in_sgpr(kc.wq[q]);
+  const double ihx2 = kc.inv_h[0] * kc.inv_h[0];
+  const double ihy2 = kc.inv_h[1] * kc.inv_h[1];
+  const double ihz2 = kc.inv_h[2] * kc.inv_h[2];
   const int lext0 = in_sgpr(a.lext[0]), lext1 = in_sgpr(a.lext[1]);
   const int nc0 = in_sgpr(a.nc[0]), nc1 = in_sgpr(a.nc[1]);
   const int npx = in_sgpr(a.plane_npx), npy = in_sgpr(a.plane_npy);
@@ -332,61 +433,71 @@ __global__ void __launch_bounds__(256)
   first = in_sgpr(first);
   end = in_sgpr(end);
   stride = in_sgpr(stride);
-  // a patch's addresses and loads (issued together at the top of the
-  // patch: carrying the next patch's loads through the computation was
-  // measured slower, at this register pressure)
+  // A patch's addresses and loads. The next patch's are issued as soon as
+  // this one's values have gone through the x contraction and arrive during
+  // its computation (a patch's loads take ~4,000 cycles, a fifth of the
+  // time it takes).
   struct PatchLoad {
-    int cx, cy, cz;
-    bool in_mesh;
-    int64_t c, base;
     uint32_t meta;
     int32_t pslot;
     uint8_t dirty;
     double u[NP];
   };
-  auto load_patch = [&](int r, PatchLoad &pl) {
-    const PlanePatch pp =
-        plane_patch(npx, npy, nzl, ymajor, r < end ? r : first);
-    pl.cx = pp.px * PX + ix;
-    pl.cy = pp.py * PY + iy;
-    pl.cz = pp.pz;
-    pl.in_mesh = r < end && cw < CPW && pl.cx < lext0 && pl.cy < lext1;
-    pl.c = pl.in_mesh ? pl.cx + (int64_t)nc0 * (pl.cy + (int64_t)nc1 * pl.cz)
-                      : 0;
-    // first node of the lane's plane (node 0 for lanes outside the mesh)
-    pl.base = pl.in_mesh ? (int64_t)pl.cx * P + sy * ((int64_t)pl.cy * P) +
-                               sz * ((int64_t)pl.cz * P + s)
-                         : 0;
-    pl.meta = meta_p[pl.c];
-    pl.pslot = slot_p[pl.c];
-    pl.dirty = (NS > 1 && liquid_p) ? dirty_p[pl.c] : 0;
+  PatchWalk walk;
+  walk.start(npx, ymajor ? nzl : npy, first, stride);
+  // addresses of lanes past the mesh are those of its last cells
+  auto load_patch = [&](PatchLoad &pl) {
+    const int py = ymajor ? walk.top : walk.mid;
+    const int pz = ymajor ? walk.mid : walk.top;
+    const int gx = min(walk.px * PX + ix, lext0 - 1);
+    const int gy = min(py * PY + iy, lext1 - 1);
+    const int64_t g = gx + (int64_t)nc0 * (gy + (int64_t)nc1 * pz);
+    const double *sp = src + (gx * P + sy * (gy * P) + sz * (pz * P + s));
+    pl.meta = meta_p[g];
+    pl.pslot = slot_p[g];
+    pl.dirty = (NS > 1 && liquid_p) ? dirty_p[g] : 0;
 #pragma unroll
     for (int yy = 0; yy < N; ++yy)
 #pragma unroll
-      for (int xx = 0; xx < N; ++xx)
-        pl.u[xx + N * yy] = src[pl.in_mesh ? pl.base + xx + sy * yy : 0];
+      for (int xx = 0; xx < N; ++xx) pl.u[xx + N * yy] = sp[xx + sy * yy];
   };
   if (first >= end) return;  // whole wavefronts
+  // JxW of the lane's points, as the host tabulates it:
+  // det * (((1 * w_x) * w_y) * w_z), w_z = w[s]; the 1-D weights are
+  // symmetric (checked on the host for Q2), so few of them differ
+  double jxw[N][N];
+  {
+    const double det = kc.det, wz = sk.wq[s];
+    double wq[N];
+#pragma unroll
+    for (int q = 0; q < N; ++q) wq[q] = kc.wq[q <= N - 1 - q ? q : N - 1 - q];
+#pragma unroll
+    for (int qx = 0; qx < N; ++qx)
+#pragma unroll
+      for (int qy = 0; qy < N; ++qy)
+        jxw[qx][qy] = det * ((wq[min(qx, qy)] * wq[max(qx, qy)]) * wz);
+  }
+  double *const xb = lds + (PK == 2 ? n_mat * kPlaneMergedLds : 0) +
+                     wave * L::wave_lds;
+  double *const myslot = xb + cw * L::cell_slots + s * SL;
+  // slot of plane n of this lane's cell
+  auto slot_of = [&](int n) { return xb + cw * L::cell_slots + n * SL; };
+  PatchLoad nxt;
+  load_patch(nxt);
+  // the lane's place in a patch's block of the patch buffer
+  const int64_t rowlen = (int64_t)npx * L::patch_nx;
+  const int64_t E_lane =
+      ((int64_t)s * npy * L::patch_ny + iy * P) * rowlen + ix * P;
   for (int r = first; r < end; r += stride) {
   wave_lds_sync();  // the previous patch's exchange reads are done
-  PatchLoad cur;
-  load_patch(r, cur);
-  const int cx = cur.cx, cy = cur.cy, cz = cur.cz;
-  const bool in_mesh = cur.in_mesh;
-  const int64_t c = cur.c;
-  const uint32_t meta0 = cur.meta;
-  const int32_t pslot32 = cur.pslot;
-  double u[NP];
-#pragma unroll
-  for (int q = 0; q < NP; ++q) u[q] = cur.u[q];
-
-  const uint32_t meta = in_mesh ? meta0 : 0u;
+  const int ppx = walk.px, ppy = ymajor ? walk.top : walk.mid,
+            ppz = ymajor ? walk.mid : walk.top;
+  const int cx = ppx * PX + ix, cy = ppy * PY + iy, cz = ppz;
+  const bool in_mesh = cw < CPW && cx < lext0 && cy < lext1;
+  const int64_t c = cx + (int64_t)nc0 * (cy + (int64_t)nc1 * cz);
+  const int32_t pslot32 = nxt.pslot;
+  const uint32_t meta = in_mesh ? nxt.meta : 0u;
   const bool act = (meta & kActive) != 0;
-  double *xb = lds + (PK == 2 ? n_mat * kPlaneMergedLds : 0) +
-               wave * L::wave_lds;
-  double *myslot = xb + lane * SL;
-  // slot of plane n of this lane's cell
-  auto slot_of = [&](int n) { return xb + (cw * N + n) * SL; };
 
   const int mid = (meta >> kMaterialShift) & 3;
   const double solidus = sk.solidus[mid], liquidus = sk.liquidus[mid];
@@ -399,11 +510,27 @@ __global__ void __launch_bounds__(256)
   ADM_GLOBAL double *lq = nullptr;
   if constexpr (NS > 1) {
     if (liquid_p && act) {
-      dirty = cur.dirty != 0;
+      dirty = nxt.dirty != 0;
       lq = liquid_p + c * N3 + NP * s;
     }
   }
   const bool rotated = act && (meta & kRotated) != 0;
+  // the stored powder of the lane's points and the cell's direction, loaded
+  // ahead of the contractions
+  double pin[NS == 3 ? NP : 1];
+  if constexpr (NS == 3) {
+#pragma unroll
+    for (int q = 0; q < NP; ++q) pin[q] = 0.0;
+    if (pw) {
+#pragma unroll
+      for (int q = 0; q < NP; ++q) pin[q] = pw[q];
+    }
+  }
+  double cs = 1.0, sn = 0.0;
+  if (rotated) {
+    cs = cos_p[c];
+    sn = sin_p[c];
+  }
 
   // ---- values: S along x, then y, in registers ---------------------------
   double v[NP];
@@ -414,15 +541,19 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int qx = 0; qx < N; ++qx) {
         if (P == 2 && qx == 1) {
-          t[qx + N * yy] = u[1 + N * yy];
+          t[qx + N * yy] = nxt.u[1 + N * yy];
           continue;
         }
-        double acc = S[qx][0] * u[N * yy];
+        double acc = S[qx][0] * nxt.u[N * yy];
 #pragma unroll
         for (int k = 1; k < N; ++k)
-          acc = __builtin_fma(S[qx][k], u[k + N * yy], acc);
+          acc = __builtin_fma(S[qx][k], nxt.u[k + N * yy], acc);
         t[qx + N * yy] = acc;
       }
+    if (r + stride < end) {
+      walk.advance();
+      load_patch(nxt);
+    }
 #pragma unroll
     for (int qy = 0; qy < N; ++qy)
 #pragma unroll
@@ -467,6 +598,7 @@ __global__ void __launch_bounds__(256)
         gz[q] = __builtin_fma(dzv[n], wn, gz[q]);
       }
   }
+  wave_lds_sync();
 
   // ---- per-point physics, one point row (fixed y) at a time --------------
   bool near = false;
@@ -486,72 +618,248 @@ __global__ void __launch_bounds__(256)
   const double *mC = mB + kMergedMax;
   const MergedBins &mbin =
       *reinterpret_cast<const MergedBins *>(mB + kMergedLds);
-  // wave-uniform fast path: one material, every point fully solid (no
-  // powder, below the solidus)
   const int mid0 = __builtin_amdgcn_readfirstlane(mid);
-  bool warm = false;
-  if constexpr (NS > 1) {
-#pragma unroll
-    for (int q = 0; q < NP; ++q) warm |= act && !(Tq[q] < solidus);
-  }
-  const bool fast =
-      !__any(warm || has_powder || (act && mid != mid0));
   // accumulators of the node plane (before the z part): Ap gathers the x
   // and y flux terms and the source, Bp the z flux
   double Ap[NP], Bp[NP];
   bool plane_liquid = false;
-  double cs = 1.0, sn = 0.0;
-  if (rotated) {
-    cs = cos_p[c];
-    sn = sin_p[c];
+
+  // x and y gradients of point (qx, qy) by the collocation derivative (the
+  // oracle's chains)
+  auto grad_xy = [&](int qx, int qy, double &gxq, double &gyq) {
+    gxq = Dc[qx][0] * Tq[N * qy];
+    gyq = Dc[qy][0] * Tq[qx];
+#pragma unroll
+    for (int k = 1; k < N; ++k) {
+      if (!(P == 2 && qx == 1 && k == 1))
+        gxq = __builtin_fma(Dc[qx][k], Tq[k + N * qy], gxq);
+      if (!(P == 2 && qy == 1 && k == 1))
+        gyq = __builtin_fma(Dc[qy][k], Tq[qx + N * k], gyq);
+    }
+  };
+  // fold a point row into the node-plane accumulators:
+  //   Ap[xx, yy] += S[qy][yy] (DcS^T w0)[xx] + DcS[qy][yy] (S^T w1)[xx]
+  //   Bp[xx, yy] += S[qy][yy] (S^T w2)[xx]
+  auto fold_row = [&](int qy, const double (&w0)[N], const double (&w1)[N],
+                      const double (&w2)[N]) {
+#pragma unroll
+    for (int xx = 0; xx < N; ++xx) {
+      double t0 = DS[0][xx] * w0[0];
+      double t1 = S[0][xx] * w1[0];
+      double t2 = S[0][xx] * w2[0];
+#pragma unroll
+      for (int q = 1; q < N; ++q) {
+        if (!(P == 2 && q == 1 && xx == 1))
+          t0 = __builtin_fma(DS[q][xx], w0[q], t0);
+        if (P == 2 && q == 1) {
+          if (xx == 1) {
+            t1 = t1 + w1[q];
+            t2 = t2 + w2[q];
+          }
+          continue;
+        }
+        t1 = __builtin_fma(S[q][xx], w1[q], t1);
+        t2 = __builtin_fma(S[q][xx], w2[q], t2);
+      }
+#pragma unroll
+      for (int yy = 0; yy < N; ++yy) {
+        const int o = xx + N * yy;
+        if (qy == 0) {
+          Ap[o] = __builtin_fma(DS[qy][yy], t1, S[qy][yy] * t0);
+          Bp[o] = S[qy][yy] * t2;
+        } else if (P == 2 && qy == 1) {
+          if (yy == 1) {
+            Ap[o] = Ap[o] + t0;
+            Bp[o] = Bp[o] + t2;
+          } else {
+            Ap[o] = __builtin_fma(DS[qy][yy], t1, Ap[o]);
+          }
+        } else {
+          Ap[o] = __builtin_fma(S[qy][yy], t0, Ap[o]);
+          Ap[o] = __builtin_fma(DS[qy][yy], t1, Ap[o]);
+          Bp[o] = __builtin_fma(S[qy][yy], t2, Bp[o]);
+        }
+      }
+    }
+  };
+
+  // One-interval form. Most planes are cold (no point at or above the
+  // solidus) and so smooth that their points lie in one interval of the
+  // merged table: the interval and its coefficients are then read once per
+  // plane instead of once per point, and nothing in the point loop branches
+  // or waits for LDS. Taken when it holds for every lane of the wavefront
+  // and every material is isotropic; without powder every point is fully
+  // solid, and with powder a mixture of solid and powder.
+  bool one = false;
+  int j1 = 0;
+  double tl = 0.0;  // left end of the plane's interval
+  if constexpr (PK == 2) {
+    j1 = merged_bin_interval(mB, mbin, Tq[0]);
+    tl = mB[j1 > 0 ? j1 - 1 : 0];
+    const double lo = j1 > 0 ? tl : -HUGE_VAL;
+    double hi = j1 < kMergedMax ? mB[j1] : HUGE_VAL;
+    if constexpr (NS > 1) hi = hi < solidus ? hi : solidus;
+    bool ok = iso;
+#pragma unroll
+    for (int q = 0; q < NP; ++q) ok = ok && Tq[q] >= lo && Tq[q] < hi;
+    one = !__any(act && !ok);
   }
-  // JxW of the lane's points as the host tabulates it:
-  // det * (((1 * w_x) * w_y) * w_z), w_z = w[s]
-  const double wz = sk.wq[s];
-  const double ihx2 = ih0 * ih0, ihy2 = ih1 * ih1, ihz2 = ih2 * ih2;
-  // SOLID: the fast path (material mid_ for every lane, ratios (1, 0, 0));
-  // otherwise the lane's own material and the phase-state update
-  auto physics = [&](auto solid_tag, int mid_, const double *mB_,
-                     const double *mC_, const MergedBins &mbin_, bool iso_,
-                     bool rot_) {
-    constexpr bool SOLID = decltype(solid_tag)::value;
-    if constexpr (SOLID && NS > 1) {
-      // every point solid: a liquid ratio held from the last evaluation
-      // goes back to zero
+  // wave-uniform solid path: one material, every point fully solid (no
+  // powder, below the solidus)
+  bool fast = false;
+  if (!one) {
+    bool warm = false;
+    if constexpr (NS > 1) {
+#pragma unroll
+      for (int q = 0; q < NP; ++q) warm |= act && !(Tq[q] < solidus);
+    }
+    fast = !__any(warm || has_powder || (act && mid != mid0));
+  }
+  auto solid_again = [&]() {
+    // every point solid: a liquid ratio held from the last evaluation goes
+    // back to zero
+    if constexpr (NS > 1) {
       if (lq && dirty) {
 #pragma unroll
         for (int q = 0; q < NP; ++q) lq[q] = 0.0;
       }
     }
-    // the stored powder of the lane's points, loaded together (one memory
-    // round trip for the plane)
-    double pin[SOLID || NS < 3 ? 1 : NP];
-    if constexpr (!SOLID && NS == 3) {
-#pragma unroll
-      for (int q = 0; q < NP; ++q) pin[q] = 0.0;
-      if (pw) {
-#pragma unroll
-        for (int q = 0; q < NP; ++q) pin[q] = pw[q];
-      }
+  };
+
+  auto one_interval = [&](auto powder_tag) {
+    constexpr bool POWDER = decltype(powder_tag)::value;
+    constexpr int row = kMergedMax * ADM_MAX_STATES * 2;
+    const double *cj = mC + j1 * (ADM_MAX_STATES * 2);
+    const double rs0 = cj[ADM_DENSITY * row], rs1 = cj[ADM_DENSITY * row + 1];
+    const double cs0 = cj[ADM_SPECIFIC_HEAT * row],
+                 cs1 = cj[ADM_SPECIFIC_HEAT * row + 1];
+    const double ks0 = cj[ADM_THERMAL_CONDUCTIVITY_X * row],
+                 ks1 = cj[ADM_THERMAL_CONDUCTIVITY_X * row + 1];
+    double rp0 = 0.0, rp1 = 0.0, cp0 = 0.0, cp1 = 0.0, kp0 = 0.0, kp1 = 0.0;
+    if constexpr (POWDER) {
+      rp0 = cj[ADM_DENSITY * row + 4], rp1 = cj[ADM_DENSITY * row + 5];
+      cp0 = cj[ADM_SPECIFIC_HEAT * row + 4];
+      cp1 = cj[ADM_SPECIFIC_HEAT * row + 5];
+      kp0 = cj[ADM_THERMAL_CONDUCTIVITY_X * row + 4];
+      kp1 = cj[ADM_THERMAL_CONDUCTIVITY_X * row + 5];
     }
-#pragma unroll
-    for (int qy = 0; qy < N; ++qy) {
+    // isotropic: the rotation K -> k (cos^2 + sin^2) in the x-y plane
+    const double rot = cs * cs + sn * sn;
+    const double ax = ihx2 * rot, ay = ihy2 * rot;
+    solid_again();
+    static_for<0, N>([&](auto qyc) {
+      constexpr int qy = decltype(qyc)::value;
       double w0[N], w1[N], w2[N];
 #pragma unroll
       for (int qx = 0; qx < N; ++qx) {
         const int q = qx + N * qy;
-        const double T = Tq[q];
-        // x and y gradients by the collocation derivative (the oracle's
-        // chains)
-        double gxq = Dc[qx][0] * Tq[N * qy];
-        double gyq = Dc[qy][0] * Tq[qx];
-#pragma unroll
-        for (int k = 1; k < N; ++k) {
-          if (!(P == 2 && qx == 1 && k == 1))
-            gxq = __builtin_fma(Dc[qx][k], Tq[k + N * qy], gxq);
-          if (!(P == 2 && qy == 1 && k == 1))
-            gyq = __builtin_fma(Dc[qy][k], Tq[qx + N * k], gyq);
+        double gxq, gyq;
+        grad_xy(qx, qy, gxq, gyq);
+        const double d = Tq[q] - tl;
+        double rho = __builtin_fma(d, rs1, rs0);
+        double cp = __builtin_fma(d, cs1, cs0);
+        double k = __builtin_fma(d, ks1, ks0);
+        if constexpr (POWDER) {
+          // l = 0: powder = min(powder, 1), solid = 1 - powder
+          const double pv = (pin[q] < 1.0) ? pin[q] : 1.0;
+          const double sv = 1.0 - pv;
+          rho = sv * rho + pv * __builtin_fma(d, rp1, rp0);
+          cp = sv * cp + pv * __builtin_fma(d, cp1, cp0);
+          k = sv * k + pv * __builtin_fma(d, kp1, kp0);
         }
+        const double irc = recip(rho * cp);
+        // the source pass reads 1 / (rho c_p) from the lane's slot
+        myslot[q] = irc;
+        const double cq = ((-irc) * jxw[qx][qy]) * k;
+        w0[qx] = cq * (gxq * ax);
+        w1[qx] = cq * (gyq * ay);
+        w2[qx] = cq * (gz[q] * ihz2);
+      }
+      fold_row(qy, w0, w1, w2);
+    });
+    if constexpr (POWDER) {
+      // powder above 1 (or not a number) is cut to 1, as stored
+      if (pw) {
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+          if (!(pin[q] < 1.0) && pin[q] != 1.0) pw[q] = 1.0;
+      }
+    }
+  };
+
+  // SOLID: the solid path (material mid_ for every lane, ratios (1, 0, 0));
+  // otherwise the lane's own material and the phase-state update
+  auto physics = [&](auto solid_tag, int mid_, const double *mB_,
+                     const double *mC_, const MergedBins &mbin_, bool iso_,
+                     bool rot_) {
+    constexpr bool SOLID = decltype(solid_tag)::value;
+    if constexpr (SOLID) solid_again();
+    // polynomial coefficients of the wave's solid material: uniform scalar
+    // loads, once per patch
+    const ADM_CONSTANT MatConst &mcst = kc.mat;
+    constexpr bool POLY1 = PK == 0 && SOLID;
+    const int order = POLY1 ? mcst.p_order : 0;
+    static_for<0, N>([&](auto qyc) {
+      constexpr int qy = decltype(qyc)::value;
+      double w0[N], w1[N], w2[N];
+      double Tr[N];
+#pragma unroll
+      for (int qx = 0; qx < N; ++qx) Tr[qx] = Tq[qx + N * qy];
+      int jr[N];
+      if constexpr (PK == 2) merged_bin_intervals<N>(mB_, mbin_, Tr, jr);
+      // update_state_ratios (source/ThermalOperator.templates.hh:227-317):
+      // the mushy division where a point of the wavefront needs it
+      double mushy[N];
+      if constexpr (!SOLID && NS > 1) {
+        bool need = false;
+#pragma unroll
+        for (int qx = 0; qx < N; ++qx) {
+          mushy[qx] = 0.0;
+          need |= !(Tr[qx] < solidus) && !(Tr[qx] > liquidus);
+        }
+        if (__any(need)) {
+#pragma unroll
+          for (int qx = 0; qx < N; ++qx)
+            mushy[qx] = (Tr[qx] - solidus) / (liquidus - solidus);
+        }
+      }
+      double rho_[N], cp_[N], kx_[N], ky_[N], kz_[N];
+      if constexpr (POLY1) {
+        // sum_i c_i T^i, state ratio 1
+        double tp[N];
+#pragma unroll
+        for (int qx = 0; qx < N; ++qx) {
+          tp[qx] = 1.0;
+          rho_[qx] = cp_[qx] = kx_[qx] = ky_[qx] = kz_[qx] = 0.0;
+        }
+#pragma unroll
+        for (int i = 0; i < ADM_MAX_POLY; ++i) {
+          if (i > order) break;
+          const double cr = mcst.poly[mid_][ADM_DENSITY][0][i];
+          const double cc = mcst.poly[mid_][ADM_SPECIFIC_HEAT][0][i];
+          const double ck =
+              mcst.poly[mid_][ADM_THERMAL_CONDUCTIVITY_X][0][i];
+          const double cy_ =
+              mcst.poly[mid_][ADM_THERMAL_CONDUCTIVITY_Y][0][i];
+          const double cz_ =
+              mcst.poly[mid_][ADM_THERMAL_CONDUCTIVITY_Z][0][i];
+#pragma unroll
+          for (int qx = 0; qx < N; ++qx) {
+            if (i > 0) tp[qx] = tp[qx] * Tr[qx];
+            rho_[qx] += cr * tp[qx];
+            cp_[qx] += cc * tp[qx];
+            kx_[qx] += ck * tp[qx];
+            ky_[qx] += cy_ * tp[qx];
+            kz_[qx] += cz_ * tp[qx];
+          }
+        }
+      }
+#pragma unroll
+      for (int qx = 0; qx < N; ++qx) {
+        const int q = qx + N * qy;
+        const double T = Tr[qx];
+        double gxq, gyq;
+        grad_xy(qx, qy, gxq, gyq);
         double r_[NS];
         double l = 0.0;
         if constexpr (SOLID || NS == 1) {
@@ -559,12 +867,10 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
           for (int k = 1; k < NS; ++k) r_[k] = 0.0;
         } else {
-          // update_state_ratios (source/ThermalOperator.templates.hh:227-317)
           double p0 = 0.0;
           if constexpr (NS == 3) p0 = pin[q];
           double pv = p0;
-          const double mushy = (T - solidus) / (liquidus - solidus);
-          l = T < solidus ? 0.0 : (T > liquidus ? 1.0 : mushy);
+          l = T < solidus ? 0.0 : (T > liquidus ? 1.0 : mushy[qx]);
           if constexpr (NS == 2) {
             r_[1] = l;
             r_[0] = 1.0 - l;
@@ -598,8 +904,13 @@ __global__ void __launch_bounds__(256)
             kzz = ev(ADM_THERMAL_CONDUCTIVITY_Z, r_);
           }
         };
-        if constexpr (PK == 2) {
-          const int j = merged_bin_interval(mB_, mbin_, T);
+        if constexpr (POLY1) {
+          irc = recip(rho_[qx] * cp_[qx]);
+          kx = kx_[qx];
+          ky = ky_[qx];
+          kzz = kz_[qx];
+        } else if constexpr (PK == 2) {
+          const int j = jr[qx];
           if constexpr (SOLID) {
             // the solid value alone: (0 + 1 X_s) + 0 X_l + 0 X_p = X_s
             const double d = T - mB_[j > 0 ? j - 1 : 0];
@@ -615,10 +926,11 @@ __global__ void __launch_bounds__(256)
         } else {
           props(typename EvalOf<PK>::type(m, mid_, T));
         }
+        myslot[q] = irc;  // for the source pass
         // -(1/rho c_p) K grad T * JxW, each component with its 1/h
-        const double jxw = det * ((wq[qx] * wq[qy]) * wz);
-        const double cq = (-irc) * jxw;
+        const double cq = (-irc) * jxw[qx][qy];
         if (rot_) {
+          const double ih0 = kc.inv_h[0], ih1 = kc.inv_h[1];
           const double gx_ = gxq * ih0, gy_ = gyq * ih1;
           const double fx = (kx * cs * cs + ky * sn * sn) * gx_ +
                             ((kx - ky) * sn * cs) * gy_;
@@ -632,47 +944,15 @@ __global__ void __launch_bounds__(256)
         }
         w2[qx] = (cq * kzz) * (gz[q] * ihz2);
       }
-      // fold the row into the node-plane accumulators:
-      //   Ap[xx, yy] += S[qy][yy] (DcS^T w0)[xx] + DcS[qy][yy] (S^T w1)[xx]
-      //   Bp[xx, yy] += S[qy][yy] (S^T w2)[xx]
-#pragma unroll
-      for (int xx = 0; xx < N; ++xx) {
-        double t0 = DS[0][xx] * w0[0];
-        double t1 = S[0][xx] * w1[0];
-        double t2 = S[0][xx] * w2[0];
-#pragma unroll
-        for (int q = 1; q < N; ++q) {
-          t0 = __builtin_fma(DS[q][xx], w0[q], t0);
-          if (P == 2 && q == 1) {
-            if (xx == 1) {
-              t1 = t1 + w1[q];
-              t2 = t2 + w2[q];
-            }
-            continue;
-          }
-          t1 = __builtin_fma(S[q][xx], w1[q], t1);
-          t2 = __builtin_fma(S[q][xx], w2[q], t2);
-        }
-#pragma unroll
-        for (int yy = 0; yy < N; ++yy) {
-          const int o = xx + N * yy;
-          if (qy == 0) {
-            Ap[o] = __builtin_fma(DS[qy][yy], t1, S[qy][yy] * t0);
-            Bp[o] = S[qy][yy] * t2;
-          } else if (P == 2 && qy == 1) {
-            if (yy == 1) Ap[o] = Ap[o] + t0;
-            Ap[o] = __builtin_fma(DS[qy][yy], t1, Ap[o]);
-            if (yy == 1) Bp[o] = Bp[o] + t2;
-          } else {
-            Ap[o] = __builtin_fma(S[qy][yy], t0, Ap[o]);
-            Ap[o] = __builtin_fma(DS[qy][yy], t1, Ap[o]);
-            Bp[o] = __builtin_fma(S[qy][yy], t2, Bp[o]);
-          }
-        }
-      }
-    }
+      fold_row(qy, w0, w1, w2);
+    });
   };
-  if (fast) {
+  if (one) {
+    if (NS == 3 && __any(has_powder))
+      one_interval(std::integral_constant<bool, NS == 3>{});
+    else
+      one_interval(std::integral_constant<bool, false>{});
+  } else if (fast) {
     // the wave's material (uniform: scalar registers, uniform LDS rows)
     const double *fB = lds + mid0 * kPlaneMergedLds;
     physics(std::integral_constant<bool, true>{}, mid0, fB, fB + kMergedMax,
@@ -684,59 +964,14 @@ __global__ void __launch_bounds__(256)
             rotated);
   }
   // heat sources, in a pass of their own over the cells that a beam can
-  // reach (few), point by point in a loop (one copy of the source code):
-  // 1/(rho c_p) of each point again from its updated state, the weighted
-  // source values through the lane's exchange slot, then
-  // Ap[xx, yy] += S[qy][yy] (S^T val)[xx]
+  // reach (few), a point row at a time: 1/(rho c_p) as the physics left it
+  // in the lane's slot, then Ap[xx, yy] += S[qy][yy] (S^T val)[xx]
   if (__any(near)) {
     wave_lds_sync();
     if (near) {
-#pragma unroll
-      for (int q = 0; q < NP; ++q) myslot[q] = Tq[q];
-#pragma unroll 1
-      for (int q = 0; q < NP; ++q) {
-        const int qx = q % N, qy = q / N;
-        const double T = myslot[q];
-        double r_[NS];
-        if constexpr (NS == 1) {
-          r_[0] = 1.0;
-        } else {
-          const double mushy = (T - solidus) / (liquidus - solidus);
-          const double l = T < solidus ? 0.0 : (T > liquidus ? 1.0 : mushy);
-          if constexpr (NS == 2) {
-            r_[1] = l;
-            r_[0] = 1.0 - l;
-          } else {
-            // the powder as this evaluation left it
-            const double pv = pw ? pw[q] : 0.0;
-            r_[1] = l;
-            r_[2] = pv;
-            r_[0] = 1.0 - l - pv;
-          }
-        }
-        double irc = 0.0;
-        auto rho_cp = [&](const auto &ev) {
-          const double density = ev(ADM_DENSITY, r_);
-          double specific_heat = ev(ADM_SPECIFIC_HEAT, r_);
-          if constexpr (NS > 1) {
-            const double is_mushy = r_[1] * r_[0];
-            if (is_mushy > 0.0) specific_heat += latent;
-          }
-          irc = recip(density * specific_heat);
-        };
-        if constexpr (PK == 2)
-          rho_cp(MergedEval(mB, mC, T, merged_bin_interval(mB, mbin, T)));
-        else
-          rho_cp(typename EvalOf<PK>::type(m, mid, T));
-        const double px = kc.origin[0] + (cx + sk.xq[qx]) * kc.h[0];
-        const double py = kc.origin[1] + (cy + sk.xq[qy]) * kc.h[1];
-        const double pz = kc.origin[2] + (cz + sk.xq[s]) * kc.h[2];
-        double qs = 0.0;
-        for (int b = 0; b < a.n_beams; ++b)
-          qs += beam_value(sbeams[b], px, py, pz, kc.log_01);
-        const double jxw = det * ((sk.wq[qx] * sk.wq[qy]) * wz);
-        myslot[q] = (qs * irc) * jxw;
-      }
+      plane_source<P>((ADM_LDS double *)myslot,
+                      (const ADM_LDS adm_beam_state *)&sbeams[0], a.n_beams,
+                      (const ADM_LDS CellConstLds *)&sk, &kc, cx, cy, cz, s);
 #pragma unroll
       for (int qy = 0; qy < N; ++qy)
 #pragma unroll
@@ -758,17 +993,24 @@ __global__ void __launch_bounds__(256)
     if (lq && s == 0 && any_liquid != dirty) dirty_p[c] = any_liquid ? 1 : 0;
   }
 
-  // ---- exchanges 2 and 3: z part, node plane s = sum over point planes --
-  // out = sum_qz S[qz][s] Ap_qz + sum_qz (Dc S)[qz][s] Bp_qz
+  // ---- exchange 2: z part, node plane s = sum over point planes ----------
+  // out = sum_qz S[qz][s] Ap_qz + sum_qz (Dc S)[qz][s] Bp_qz, the two
+  // parts in a buffer each
   double out[NP];
   wave_lds_sync();
 #pragma unroll
-  for (int q = 0; q < NP; ++q) myslot[q] = Ap[q];
+  for (int q = 0; q < NP; ++q) {
+    myslot[q] = Ap[q];
+    myslot[L::exchange + q] = Bp[q];
+  }
   wave_lds_sync();
   {
-    double sc[N];
+    double sc[N], dc[N];
 #pragma unroll
-    for (int k = 0; k < N; ++k) sc[k] = sk.S[k][s];
+    for (int k = 0; k < N; ++k) {
+      sc[k] = sk.S[k][s];
+      dc[k] = sk.Dc[k][s];  // (Dc S)[k][s]
+    }
 #pragma unroll
     for (int q = 0; q < NP; ++q) out[q] = sc[0] * slot_of(0)[q];
 #pragma unroll
@@ -776,20 +1018,11 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int q = 0; q < NP; ++q)
         out[q] = __builtin_fma(sc[k], slot_of(k)[q], out[q]);
-  }
-  wave_lds_sync();
-#pragma unroll
-  for (int q = 0; q < NP; ++q) myslot[q] = Bp[q];
-  wave_lds_sync();
-  {
-    double dc[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k) dc[k] = sk.Dc[k][s];  // (Dc S)[k][s]
 #pragma unroll
     for (int k = 0; k < N; ++k)
 #pragma unroll
       for (int q = 0; q < NP; ++q)
-        out[q] = __builtin_fma(dc[k], slot_of(k)[q], out[q]);
+        out[q] = __builtin_fma(dc[k], slot_of(k)[L::exchange + q], out[q]);
   }
   if (!act) {
 #pragma unroll
@@ -810,6 +1043,10 @@ __global__ void __launch_bounds__(256)
     const double o = __shfl_down(out[xx], N * PX);
     if (iy + 1 < PY) out[xx + N * P] += o;
   }
+  // the next patch's loads have arrived by now: waiting for them here keeps
+  // their wait from including the stores below
+#pragma unroll
+  for (int q = 0; q < NP; ++q) asm volatile("" : "+v"(nxt.u[q]));
   if (in_mesh) {
   // the patch's node sums, every node of the patch once, into its slots
   // of the patch buffer (plain stores; the gather kernel adds the slots of
@@ -817,12 +1054,10 @@ __global__ void __launch_bounds__(256)
   // patch buffer layout [cell layer][plane][patch y][node y][patch x]
   // [node x]: a node row of one plane runs through the patches of a row
   // contiguously, which the gather pass reads along x
-  const PlanePatch pp = plane_patch(npx, npy, nzl, ymajor, r);
-  const int64_t rowlen = (int64_t)npx * L::patch_nx;
   double *E = patch_E +
-              ((((int64_t)pp.pz * N + s) * npy + pp.py) * L::patch_ny +
-               iy * P) * rowlen +
-              (int64_t)pp.px * L::patch_nx + ix * P;
+              (((int64_t)ppz * N * npy + ppy) * L::patch_ny * rowlen +
+               (int64_t)ppx * L::patch_nx) +
+              E_lane;
 #pragma unroll
   for (int yy = 0; yy < N; ++yy)
 #pragma unroll
