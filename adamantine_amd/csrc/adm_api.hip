@@ -377,6 +377,12 @@ void Context::build_merged_tables() {
   for (int mid = 0; mid < mc.n_materials; ++mid) mc.bins[mid].maxc = maxc;
 }
 
+bool Context::all_isotropic() const {
+  for (int mid = 0; mid < kc.mat.n_materials; ++mid)
+    if (!kc.mat.isotropic[mid]) return false;
+  return true;
+}
+
 int Context::property_kind() const {
   if (!use_table) return 0;
   return kc.mat.merged_ok ? 2 : 1;
@@ -513,12 +519,11 @@ Context::Context(const adm_problem_desc &d) {
       use_plane = false;
       plane_tables_ok = false;
     } else {
-      // Dc S inherits Dc's antisymmetry, and its rows differentiate a
-      // constant to zero; its last bits are made to
-      kc.DcS[0][1] = -(kc.DcS[0][0] + kc.DcS[0][2]);
+      // Dc S inherits Dc's antisymmetry; its last bits are made to (the last
+      // row's are the ones that differentiate a constant closest to zero)
       kc.DcS[1][1] = 0.0;
       kc.DcS[1][2] = -kc.DcS[1][0];
-      for (int i = 0; i < 3; ++i) kc.DcS[2][i] = -kc.DcS[0][2 - i];
+      for (int i = 0; i < 3; ++i) kc.DcS[0][i] = -kc.DcS[2][2 - i];
     }
   }
   det = 1.0;
@@ -535,6 +540,9 @@ Context::Context(const adm_problem_desc &d) {
   }
   for (int q = 0; q < n1; ++q) kc.wq[q] = wq[q];
   kc.det = det;
+  for (int k = 0; k < 3; ++k) kc.inv_h2[k] = kc.inv_h[k] * kc.inv_h[k];
+  for (int x = 0; x < n1; ++x)
+    for (int y = 0; y < n1; ++y) kc.jxy[x][y] = det * (wq[x] * wq[y]);
   for (int q = 0; q < nq; ++q) {
     double w = 1.0;
     int r = q;
@@ -1329,6 +1337,21 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
     ac.n_rows = ac.plane_npx * ac.plane_npy * lim[2];
     const int64_t slots = p == 1 ? PlaneLanes<1>::patch_nodes
                                  : PlaneLanes<2>::patch_nodes;
+    if (ac.beam_table) {
+      // the beams of a captured loop are not known here
+      for (int d = 0; d < 3; ++d) {
+        ac.reach_lo[d] = -(1 << 30);
+        ac.reach_hi[d] = 1 << 30;
+      }
+    } else {
+      beam_reach(ac.beams, ac.n_beams, kc.origin, kc.inv_h, ac.reach_lo,
+                 ac.reach_hi);
+    }
+    const bool iso = all_isotropic();
+    ac.plane_wave_lds = p == 1 ? (iso ? PlaneLanes<1>::wave_lds
+                                      : PlaneLanes<1>::wave_lds_aniso)
+                               : (iso ? PlaneLanes<2>::wave_lds
+                                      : PlaneLanes<2>::wave_lds_aniso);
     ac.plane_E_stride = (int64_t)ac.n_rows * slots;
     if (patch) {
       if ((size_t)ac.plane_E_stride * M > kNoAllocScratchDoubles)

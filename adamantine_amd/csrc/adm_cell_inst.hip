@@ -25,7 +25,7 @@ template <int P, int NS, int PK>
 void launch_plane(const CellArgs &a, const double *src, double *dst,
                   int64_t n_blocks, size_t lds_bytes, unsigned n_members,
                   int waves, hipStream_t s) {
-  const size_t xbytes = sizeof(double) * waves * PlaneLanes<P>::wave_lds;
+  const size_t xbytes = sizeof(double) * waves * a.plane_wave_lds;
   hipLaunchKernelGGL((plane_kernel<P, NS, PK>), dim3((unsigned)n_blocks,
                      n_members), dim3(64 * waves), lds_bytes + xbytes, s, a,
                      src, dst);

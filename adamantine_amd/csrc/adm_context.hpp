@@ -158,6 +158,7 @@ struct Context {
   FaceArgs face_args() const;
   void build_merged_tables();
   int property_kind() const;
+  bool all_isotropic() const;
   // patch: the plane kernel's patch buffer for this call (NULL: the
   // context's own, grown on demand)
   void apply(const double *src, double *dst, int add, hipStream_t s,

@@ -88,6 +88,8 @@ struct KConst {
   double jxw[kMaxQ];         // det * ((1 * wq[x]) * wq[y]) * wq[z]
   double fjxw[3][kMaxFQ];    // face JxW per normal direction
   double h[3], inv_h[3], origin[3];
+  double inv_h2[3];          // inv_h^2
+  double jxy[kMaxN][kMaxN];  // det * (wq[x] * wq[y])
   int32_t n_boundary_ids;
   int32_t boundary_type[ADM_MAX_BOUNDARY_IDS];
   int32_t adiabatic_only;
@@ -178,6 +180,8 @@ struct CellArgs {
   // patch buffer the kernel writes its nodes' sums to (plane_slots doubles
   // per patch, plane_E_stride per ensemble member) for the gather kernel
   int32_t plane_npx, plane_npy;
+  int32_t plane_wave_lds;  // doubles of LDS per wavefront
+  int32_t reach_lo[3], reach_hi[3];  // beam_reach of the launch's beams
   double *plane_E;
   int64_t plane_E_stride;
 };
@@ -517,6 +521,51 @@ __device__ __forceinline__ double beam_value(const adm_beam_state &s, double x,
   return 1.0 * s.alpha * exp(exponent) * factor;
 }
 
+// qs[i] += beam_value at (x[i], y, z) for M points of a row, by selects: the
+// exponentials of the points overlap. The same bits as beam_value (a point
+// cut off adds zero). The beam is the same for every lane.
+template <int M>
+__device__ __forceinline__ void beam_values(const adm_beam_state &s,
+                                            const double (&x)[M], double y,
+                                            double z, double log_01,
+                                            double (&qs)[M]) {
+  const int type = __builtin_amdgcn_readfirstlane(s.type);
+  if (type == ADM_SOURCE_CUBE || __builtin_amdgcn_readfirstlane(s.rotated)) {
+#pragma unroll
+    for (int i = 0; i < M; ++i) qs[i] += beam_value(s, x[i], y, z, log_01);
+    return;
+  }
+  const double zc = z - s.center[2], dy = y - s.center[1];
+  const bool deep = zc + s.depth < 0.0;
+  double factor = 1.0;
+  if (type != ADM_SOURCE_GOLDAK) {
+    const double z_rel = zc * s.inv_depth;
+    factor = z_rel * z_rel;
+    factor *= -3.0;
+    factor -= z_rel;
+    factor -= z_rel;
+    factor += 1.0;
+  }
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    const double dx = x[i] - s.center[0];
+    double xy2 = dx * dx;
+    xy2 += dy * dy;
+    const bool off = deep || 5. * s.radius_squared - xy2 < 0.;
+    double exponent;
+    if (type == ADM_SOURCE_GOLDAK) {
+      exponent = zc * zc * s.inv_depth_squared;
+      exponent += xy2 * s.inv_radius_squared;
+      exponent *= -3.0;
+    } else {
+      exponent = log_01 * xy2;
+      exponent *= s.inv_radius_squared;
+    }
+    const double v = 1.0 * s.alpha * exp(exponent) * factor;
+    qs[i] += off ? 0.0 : v;
+  }
+}
+
 // True if beam s can be non-zero somewhere in the box [lo, hi] (the cut-offs
 // z + depth < 0 and |xy|^2 > 5 R^2 of the reference, or the cube's box).
 __host__ __device__ __forceinline__ bool beam_may_touch(
@@ -560,6 +609,42 @@ __host__ __device__ __forceinline__ bool beam_may_touch(
   }
   // generous margin: a false positive only costs the evaluation
   return !(d2 > 5.0 * s.radius_squared * (1.0 + 1e-6));
+}
+
+// A box of cells [lo, hi] outside which beam_may_touch is false for every
+// beam: the cut-offs in cell units, a cell wider on each side (every cell
+// for a rotated source or numbers that do not compare).
+inline void beam_reach(const adm_beam_state *beams, int n_beams,
+                       const double (&origin)[3], const double (&inv_h)[3],
+                       int32_t (&lo)[3], int32_t (&hi)[3]) {
+  constexpr int32_t big = 1 << 30;
+  for (int d = 0; d < 3; ++d) {
+    lo[d] = big;
+    hi[d] = -big;
+  }
+  for (int b = 0; b < n_beams; ++b) {
+    const adm_beam_state &s = beams[b];
+    const bool cube = s.type == ADM_SOURCE_CUBE;
+    if (cube && !s.on) continue;
+    const double r = sqrt(5.0 * s.radius_squared) * (1.0 + 1e-5);
+    for (int d = 0; d < 3; ++d) {
+      const double x0 = cube ? s.cube_min[d]
+                             : (d < 2 ? s.center[d] - r
+                                      : s.center[2] - s.depth);
+      const double x1 = cube ? s.cube_max[d]
+                             : (d < 2 ? s.center[d] + r : HUGE_VAL);
+      const double c0 = (x0 - origin[d]) * inv_h[d] - 2.001;
+      const double c1 = (x1 - origin[d]) * inv_h[d] + 2.001;
+      // out of range or not a number: no limit
+      const bool all = !cube && s.rotated;
+      const int32_t i0 =
+          !all && c0 > -1e9 ? (c0 < 1e9 ? (int32_t)c0 : big) : -big;
+      const int32_t i1 =
+          !all && c1 < 1e9 ? (c1 > -1e9 ? (int32_t)c1 : -big) : big;
+      lo[d] = i0 < lo[d] ? i0 : lo[d];
+      hi[d] = i1 > hi[d] ? i1 : hi[d];
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -39,13 +39,19 @@
 //    a point loop without branches or LDS reads (see there);
 //  - the next patch's loads are issued a patch ahead;
 //  - a row's interval look-ups advance together;
-//  - the heat source sits behind a call and scalar constants that follow
-//    from symmetry are not held twice, so that nothing spills: one spilled
-//    register's reload waits for the loads in flight before it;
+//  - the other wavefronts work in two steps with the points' properties in
+//    LDS between them (see there), the heat source sits behind a call and
+//    scalar constants that follow from symmetry are not held twice, so that
+//    nothing spills: one spilled register's reload waits for the loads in
+//    flight before it;
 //  - the two parts of the integration share one exchange.
 // 128x64x32 Q2, per application (plane + gather + face kernels): 100.4 us
-// before, 77.7 us with these; 64 members of 64x32x16, per RK4 step: 3.17 ms
-// before, 2.32 ms.
+// before, 76.9 us with these; 64 members of 64x32x16, per RK4 step: 3.17 ms
+// before, 2.39 ms; Q1 101x67x33: 38.6 us before, 28.6 us. What is left of the
+// large launch is its slowest wavefront (melt under the beam: 133,000 cycles
+// against a mean of 87,000). Handing patches out by a counter instead of a
+// fixed share took 73 us there, but the counter's round trip cost the short
+// Q1 patches 10 % and batched launches 2 %.
 // Wavefronts that are solid across several intervals (one material, no
 // powder, below the solidus) take a path of their own: the mixtures reduce
 // to the solid value (the reference adds the other states with a zero ratio,
@@ -74,8 +80,14 @@ struct PlaneLanes {
   // slots of every lane's cell, including the partial cell of the lanes
   // past the last whole one (Q2: lane 63 addresses cell 21's planes)
   static constexpr int exchange = ((64 + N - 1) / N) * cell_slots;
-  // two buffers: the two parts of the integration are exchanged at once
+  // two buffers: the two parts of the integration are exchanged at once.
+  // Between the exchanges the same words hold values of the lane's points,
+  // [point][lane]: two arrays, or three where a material is anisotropic
+  static constexpr int points = 64 * NP;
   static constexpr int wave_lds = 2 * exchange;
+  static constexpr int wave_lds_aniso =
+      wave_lds > 3 * points ? wave_lds : 3 * points;
+  static_assert(wave_lds >= 2 * points, "point arrays");
   // nodes of a patch: (P PX + 1) x (P PY + 1) per plane, N planes; the
   // patch buffer holds one double per node, [plane][y][x]
   static constexpr int patch_nx = P * PX + 1, patch_ny = P * PY + 1;
@@ -94,41 +106,41 @@ constexpr int kPlaneMergedLds =
     kMergedLds + (int)(sizeof(MergedBins) / sizeof(double));
 static_assert(sizeof(MergedBins) % sizeof(double) == 0, "bins layout");
 
-// Patch coordinates of a wavefront's patch index r in a plane launch of
-// npx x npy patches per cell layer and nz layers: x fastest, then y, then
-// the cell layer; or (ymajor) x fastest, then the cell layer, then y -- the
-// order in which the XCD-aware launch hands each XCD one contiguous range,
-// so that every XCD takes a slab of patch rows through all the layers and as
-// many of the slow layers (powder, melt) as the others. The wavefront's next
-// patch is a fixed stride on: the stride is divided once and the coordinates
-// then advance by additions and carries.
-struct PatchWalk {
-  int px, mid, top;        // coordinates: x, then the middle and slow ones
-  int dx, dm, dt;          // the stride's
-  int npx, nmid;
-  __device__ __forceinline__ void start(int npx_, int nmid_, int r,
-                                        int stride) {
-    npx = npx_;
-    nmid = nmid_;
-    px = r % npx;
-    mid = (r / npx) % nmid;
-    top = r / npx / nmid;
-    dx = stride % npx;
-    dm = (stride / npx) % nmid;
-    dt = stride / npx / nmid;
+// Quotient and remainder by a divisor used many times: with
+// m = floor(2^32 / d) (2^32 - 1 for d = 1) the high word of r m is the
+// quotient or one less for every r < 2^31.
+struct FastDiv {
+  uint32_t d, m;
+  __device__ __forceinline__ explicit FastDiv(uint32_t d_)
+      : d(d_), m(d_ > 1 ? (uint32_t)(0x100000000ull / d_) : 0xffffffffu) {}
+  __device__ __forceinline__ uint32_t div(uint32_t r, uint32_t &rem) const {
+    uint32_t q = (uint32_t)(((uint64_t)r * m) >> 32);
+    rem = r - q * d;
+    if (rem >= d) {
+      ++q;
+      rem -= d;
+    }
+    return q;
   }
-  __device__ __forceinline__ void advance() {
-    px += dx;
-    mid += dm;
-    top += dt;
-    if (px >= npx) {
-      px -= npx;
-      ++mid;
-    }
-    if (mid >= nmid) {
-      mid -= nmid;
-      ++top;
-    }
+};
+
+// Coordinates of patch index r in a plane launch of npx x npy patches per
+// cell layer and nz layers: x fastest, then y, then the cell layer; or
+// (ymajor) x fastest, then the cell layer, then y -- the order in which the
+// XCD-aware launch hands each XCD one contiguous range, so that every XCD
+// takes a slab of patch rows through all the layers and as many of the slow
+// layers (powder, melt) as the others.
+struct PatchAt {
+  int px, py, pz;
+  __device__ __forceinline__ PatchAt(const FastDiv &by_npx,
+                                     const FastDiv &by_mid, bool ymajor,
+                                     int r) {
+    uint32_t x, mid;
+    const uint32_t t = by_npx.div((uint32_t)r, x);
+    const uint32_t top = by_mid.div(t, mid);
+    px = (int)x;
+    py = (int)(ymajor ? top : mid);
+    pz = (int)(ymajor ? mid : top);
   }
 };
 
@@ -196,8 +208,8 @@ __device__ __forceinline__ T in_sgpr(T x) {
   return x;
 }
 
-// Heat-source values of one lane's point plane: slot[q], 1/(rho c_p) of the
-// point on entry, becomes source * 1/(rho c_p) * JxW. Not inlined: few
+// Heat-source values of one lane's point plane: slot[64 q], 1/(rho c_p) of
+// point q on entry, becomes source * 1/(rho c_p) * JxW. Not inlined: few
 // wavefronts come here, and the exponential's constants would otherwise be
 // kept in registers through the whole patch loop (28 registers that it then
 // spills).
@@ -209,25 +221,23 @@ static __device__ __attribute__((noinline)) void plane_source(
     int cy, int cz, int s) {
   constexpr int N = P + 1;
   const double pz = kc->origin[2] + (cz + sk->xq[s]) * kc->h[2];
-  const double det = kc->det, wz = sk->wq[s];
 #pragma unroll 1
   for (int qy = 0; qy < N; ++qy) {
     const double py = kc->origin[1] + (cy + sk->xq[qy]) * kc->h[1];
-    double qs[N];
-#pragma unroll
-    for (int qx = 0; qx < N; ++qx) qs[qx] = 0.0;
-#pragma unroll 1
-    for (int b = 0; b < n_beams; ++b)
-#pragma unroll
-      for (int qx = 0; qx < N; ++qx) {
-        const double px = kc->origin[0] + (cx + sk->xq[qx]) * kc->h[0];
-        qs[qx] += beam_value(*(const adm_beam_state *)(beams + b), px, py, pz,
-                             kc->log_01);
-      }
+    double px[N], qs[N];
 #pragma unroll
     for (int qx = 0; qx < N; ++qx) {
-      const double jxw = det * ((sk->wq[qx] * sk->wq[qy]) * wz);
-      slot[qx + N * qy] = (qs[qx] * slot[qx + N * qy]) * jxw;
+      px[qx] = kc->origin[0] + (cx + sk->xq[qx]) * kc->h[0];
+      qs[qx] = 0.0;
+    }
+#pragma unroll 1
+    for (int b = 0; b < n_beams; ++b)
+      beam_values<N>(*(const adm_beam_state *)(beams + b), px, py, pz,
+                     kc->log_01, qs);
+#pragma unroll
+    for (int qx = 0; qx < N; ++qx) {
+      const int q = qx + N * qy;
+      slot[64 * q] = (qs[qx] * slot[64 * q]) * kc->jxy[qx][qy];  // w_z: later
     }
   }
 }
@@ -267,123 +277,6 @@ __global__ void __launch_bounds__(256)
   extern __shared__ double lds[];
   __shared__ adm_beam_state sbeams[ADM_MAX_BEAMS];
   __shared__ CellConstLds sk;
-  const int n_mat = kc.mat.n_materials;
-
-  {
-    constexpr int words = sizeof(adm_beam_state) * ADM_MAX_BEAMS / 8;
-    const int tid = threadIdx.x;
-    const adm_beam_state *bsrc = a.beams;
-    int bslot = 0;
-    if (a.beam_table) {
-      bslot = *as_global(a.beam_slot);
-      bslot = bslot < 0 ? 0
-                        : (bslot < a.beam_table_len ? bslot
-                                                    : a.beam_table_len - 1);
-      bsrc = a.beam_table + (int64_t)bslot * ADM_MAX_BEAMS;
-    }
-    if (tid < words)
-      reinterpret_cast<uint64_t *>(sbeams)[tid] =
-          reinterpret_cast<const uint64_t *>(bsrc)[tid];
-    constexpr int nn = kMaxN * kMaxN;
-    if (tid < nn) {
-      (&sk.S[0][0])[tid] = (&kc.S[0][0])[tid];
-      (&sk.Dc[0][0])[tid] = (&kc.DcS[0][0])[tid];  // Dc S (z direction)
-    } else if (tid < nn + kMaxN) {
-      sk.xq[tid - nn] = kc.xq[tid - nn];
-      sk.wq[tid - nn] = kc.wq[tid - nn];
-    } else if (tid >= 64 && tid < 64 + ADM_MAX_MATERIALS) {
-      const int k = tid - 64;
-      sk.solidus[k] = kc.mat.prop[k][ADM_SOLIDUS];
-      sk.liquidus[k] = kc.mat.prop[k][ADM_LIQUIDUS];
-      sk.latent[k] = kc.mat.latent_factor[k];
-      sk.iso[k] = kc.mat.isotropic[k] ? 1.0 : 0.0;
-    }
-    if constexpr (PK == 2) {
-      const int total = n_mat * kPlaneMergedLds;
-      for (int i = tid; i < total; i += blockDim.x) {
-        const int mm = i / kPlaneMergedLds, k = i % kPlaneMergedLds;
-        lds[i] = k < kMergedLds
-                     ? (&kc.mat.merged[mm].B[0])[k]
-                     : reinterpret_cast<const ADM_CONSTANT double *>(
-                           &kc.mat.bins[mm])[k - kMergedLds];
-      }
-    }
-    __syncthreads();
-    if (mb && tid < ADM_MAX_BEAMS) {
-      double pmod = a.beam_pmod[tid], den = a.beam_den[tid];
-      if (a.beam_pd_table) {
-        const double *pd =
-            a.beam_pd_table + (int64_t)bslot * 2 * ADM_MAX_BEAMS;
-        pmod = pd[tid];
-        den = pd[ADM_MAX_BEAMS + tid];
-      }
-      sbeams[tid].alpha = member_alpha(sbeams[tid], mb->beam_gain[tid], pmod,
-                                       den, kc.log_01);
-    }
-    if (mb) __syncthreads();
-  }
-  int sources_on = a.sources_on;
-  if (a.beam_table) {
-    sources_on = 0;
-    for (int b = 0; b < a.n_beams; ++b) sources_on |= sbeams[b].on ? 1 : 0;
-  }
-  // uniform constants, in scalar registers for the whole patch loop:
-  // in-plane shape values, collocation derivative, DcS, geometry and the
-  // kernel arguments the loop reads. For Q2 the host has checked that the
-  // middle Gauss point is the middle node (S row 1 = (0, 1, 0)), that S is
-  // symmetric under reflection except S[2][1] and that Dc is antisymmetric
-  // with Dc[1][1] = 0, bit for bit: S and Dc then take 8 scalar values
-  // instead of 18, and the middle rows' products by 0 and 1 are skipped,
-  // which leaves every sum as the generic chain gives it (x + 0 = x for the
-  // finite temperatures here).
-  double S[N][N], Dc[N][N], DS[N][N];
-  if constexpr (P == 2) {
-    const double s00 = in_sgpr(kc.S[0][0]), s01 = in_sgpr(kc.S[0][1]),
-                 s02 = in_sgpr(kc.S[0][2]), s21 = in_sgpr(kc.S[2][1]);
-    const double d00 = in_sgpr(kc.Dc[0][0]), d01 = in_sgpr(kc.Dc[0][1]),
-                 d02 = in_sgpr(kc.Dc[0][2]), d10 = in_sgpr(kc.Dc[1][0]);
-    S[0][0] = s00;
-    S[0][1] = s01;
-    S[0][2] = s02;
-    S[1][0] = -0.0;
-    S[1][1] = 1.0;
-    S[1][2] = 0.0;
-    S[2][0] = s02;
-    S[2][1] = s21;
-    S[2][2] = s00;
-    Dc[0][0] = d00;
-    Dc[0][1] = d01;
-    Dc[0][2] = d02;
-    Dc[1][0] = d10;
-    Dc[1][1] = 0.0;
-    Dc[1][2] = -d10;
-    Dc[2][0] = -d02;
-    Dc[2][1] = -d01;
-    Dc[2][2] = -d00;
-    const double e00 = in_sgpr(kc.DcS[0][0]), e01 = in_sgpr(kc.DcS[0][1]),
-                 e02 = in_sgpr(kc.DcS[0][2]), e10 = in_sgpr(kc.DcS[1][0]);
-    DS[0][0] = e00;
-    DS[0][1] = e01;
-    DS[0][2] = e02;
-    DS[1][0] = e10;
-    DS[1][1] = 0.0;
-    DS[1][2] = -e10;
-    DS[2][0] = -e02;
-    DS[2][1] = -e01;
-    DS[2][2] = -e00;
-  } else {
-#pragma unroll
-    for (int q = 0; q < N; ++q)
-#pragma unroll
-      for (int k = 0; k < N; ++k) {
-        S[q][k] = in_sgpr(kc.S[q][k]);
-        Dc[q][k] = in_sgpr(kc.Dc[q][k]);
-        DS[q][k] = in_sgpr(kc.DcS[q][k]);
-      }
-  }
-  const double ihx2 = kc.inv_h[0] * kc.inv_h[0];
-  const double ihy2 = kc.inv_h[1] * kc.inv_h[1];
-  const double ihz2 = kc.inv_h[2] * kc.inv_h[2];
   const int lext0 = in_sgpr(a.lext[0]), lext1 = in_sgpr(a.lext[1]);
   const int nc0 = in_sgpr(a.nc[0]), nc1 = in_sgpr(a.nc[1]);
   const int npx = in_sgpr(a.plane_npx), npy = in_sgpr(a.plane_npy);
@@ -443,16 +336,13 @@ __global__ void __launch_bounds__(256)
     uint8_t dirty;
     double u[NP];
   };
-  PatchWalk walk;
-  walk.start(npx, ymajor ? nzl : npy, first, stride);
+  const FastDiv by_npx(npx), by_mid(ymajor ? nzl : npy);
   // addresses of lanes past the mesh are those of its last cells
-  auto load_patch = [&](PatchLoad &pl) {
-    const int py = ymajor ? walk.top : walk.mid;
-    const int pz = ymajor ? walk.mid : walk.top;
-    const int gx = min(walk.px * PX + ix, lext0 - 1);
-    const int gy = min(py * PY + iy, lext1 - 1);
-    const int64_t g = gx + (int64_t)nc0 * (gy + (int64_t)nc1 * pz);
-    const double *sp = src + (gx * P + sy * (gy * P) + sz * (pz * P + s));
+  auto load_patch = [&](const PatchAt &at, PatchLoad &pl) {
+    const int gx = min(at.px * PX + ix, lext0 - 1);
+    const int gy = min(at.py * PY + iy, lext1 - 1);
+    const int64_t g = gx + (int64_t)nc0 * (gy + (int64_t)nc1 * at.pz);
+    const double *sp = src + (gx * P + sy * (gy * P) + sz * (at.pz * P + s));
     pl.meta = meta_p[g];
     pl.pslot = slot_p[g];
     pl.dirty = (NS > 1 && liquid_p) ? dirty_p[g] : 0;
@@ -461,37 +351,212 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int xx = 0; xx < N; ++xx) pl.u[xx + N * yy] = sp[xx + sy * yy];
   };
-  if (first >= end) return;  // whole wavefronts
-  // JxW of the lane's points, as the host tabulates it:
-  // det * (((1 * w_x) * w_y) * w_z), w_z = w[s]; the 1-D weights are
-  // symmetric (checked on the host for Q2), so few of them differ
-  double jxw[N][N];
+  // What depends on the loaded cell words: the stored powder of the lane's
+  // points and the cell's direction. Loaded before the stores of the patch
+  // ahead, to arrive by the time of the point work.
+  struct PatchMore {
+    double pin[NS == 3 ? NP : 1];
+    double cs, sn;
+  };
+  auto load_more = [&](const PatchAt &at, const PatchLoad &pl,
+                       PatchMore &pm) {
+    const int gx = at.px * PX + ix, gy = at.py * PY + iy;
+    const bool in = cw < CPW && gx < lext0 && gy < lext1;
+    const uint32_t w = in && (pl.meta & kActive) ? pl.meta : 0u;
+    pm.cs = 1.0;
+    pm.sn = 0.0;
+    if (w & kRotated) {
+      const int64_t g = gx + (int64_t)nc0 * (gy + (int64_t)nc1 * at.pz);
+      pm.cs = cos_p[g];
+      pm.sn = sin_p[g];
+    }
+#pragma unroll
+    for (int q = 0; q < (NS == 3 ? NP : 1); ++q) pm.pin[q] = 0.0;
+    if constexpr (NS == 3) {
+      if (w & kHasPowder) {
+        const ADM_GLOBAL double *sp =
+            powder_p + (int64_t)pl.pslot * N3 + NP * s;
+#pragma unroll
+        for (int q = 0; q < NP; ++q) pm.pin[q] = sp[q];
+      }
+    }
+  };
+  PatchLoad nxt;
+  PatchMore more;
+  // a wavefront without a patch loads the first one's (and leaves below)
+  PatchAt nat(by_npx, by_mid, ymajor, first < end ? first : 0);
+  load_patch(nat, nxt);
+  const int n_mat = kc.mat.n_materials;
+
+  // Block prologue: beams, constants and merged tables into LDS. It is a
+  // good part of a launch with one patch per wavefront, so its loads (after
+  // the first patch's, above) are all issued before the first is waited for.
   {
-    const double det = kc.det, wz = sk.wq[s];
-    double wq[N];
+    constexpr int words = sizeof(adm_beam_state) * ADM_MAX_BEAMS / 8;
+    constexpr int nn = kMaxN * kMaxN, nm = ADM_MAX_MATERIALS;
+    static_assert(words <= 128 && 2 * nn + 2 * kMaxN + 4 * nm <= 128,
+                  "one word per lane of the smallest block");
+    static_assert(sizeof(CellConstLds) ==
+                      sizeof(double) * (2 * nn + 2 * kMaxN + 4 * nm),
+                  "staged in the order of its members");
+    const int tid = threadIdx.x;
+    const adm_beam_state *bsrc = a.beams;
+    int bslot = 0;
+    if (a.beam_table) {
+      bslot = *as_global(a.beam_slot);
+      bslot = bslot < 0 ? 0
+                        : (bslot < a.beam_table_len ? bslot
+                                                    : a.beam_table_len - 1);
+      bsrc = a.beam_table + (int64_t)bslot * ADM_MAX_BEAMS;
+    }
+    const uint64_t beam_word =
+        reinterpret_cast<const uint64_t *>(bsrc)[min(tid, words - 1)];
+    const int km = tid & (nm - 1);  // material of the lanes below
+    const ADM_CONSTANT double *cp = &kc.S[0][0] + min(tid, nn - 1);
+    if (tid >= nn) cp = &kc.DcS[0][0] + (tid - nn);  // Dc S (z direction)
+    if (tid >= 2 * nn) cp = &kc.xq[0] + (tid - 2 * nn);
+    if (tid >= 2 * nn + kMaxN) cp = &kc.wq[0] + (tid - 2 * nn - kMaxN);
+    constexpr int n1d = 2 * nn + 2 * kMaxN;
+    static_assert(n1d % nm == 0, "material index of a lane");
+    if (tid >= n1d) cp = &kc.mat.prop[km][ADM_SOLIDUS];
+    if (tid >= n1d + nm) cp = &kc.mat.prop[km][ADM_LIQUIDUS];
+    if (tid >= n1d + 2 * nm) cp = &kc.mat.latent_factor[km];
+    const double const_word = *cp;
+    const double iso_word = kc.mat.isotropic[km] ? 1.0 : 0.0;
+    double gain = 0.0, pmod = 0.0, den = 1.0;
+    if (mb && tid < ADM_MAX_BEAMS) {
+      gain = mb->beam_gain[tid];
+      pmod = a.beam_pmod[tid];
+      den = a.beam_den[tid];
+      if (a.beam_pd_table) {
+        const double *pd =
+            a.beam_pd_table + (int64_t)bslot * 2 * ADM_MAX_BEAMS;
+        pmod = pd[tid];
+        den = pd[ADM_MAX_BEAMS + tid];
+      }
+    }
+    if constexpr (PK == 2) {
+      for (int mm = 0; mm < n_mat; ++mm) {
+        const ADM_CONSTANT double *tab = &kc.mat.merged[mm].B[0];
+        const ADM_CONSTANT double *bin =
+            reinterpret_cast<const ADM_CONSTANT double *>(&kc.mat.bins[mm]) -
+            kMergedLds;
+        double *out = lds + mm * kPlaneMergedLds;
+        constexpr int R = 4;  // words per lane and round
+        for (int k0 = tid; k0 < kPlaneMergedLds; k0 += R * blockDim.x) {
+          double w[R];
 #pragma unroll
-    for (int q = 0; q < N; ++q) wq[q] = kc.wq[q <= N - 1 - q ? q : N - 1 - q];
+          for (int i = 0; i < R; ++i) {
+            const int k = min(k0 + i * (int)blockDim.x, kPlaneMergedLds - 1);
+            w[i] = (k < kMergedLds ? tab : bin)[k];
+          }
 #pragma unroll
-    for (int qx = 0; qx < N; ++qx)
-#pragma unroll
-      for (int qy = 0; qy < N; ++qy)
-        jxw[qx][qy] = det * ((wq[min(qx, qy)] * wq[max(qx, qy)]) * wz);
+          for (int i = 0; i < R; ++i) {
+            const int k = k0 + i * (int)blockDim.x;
+            if (k < kPlaneMergedLds) out[k] = w[i];
+          }
+        }
+      }
+    }
+    if (tid < words) reinterpret_cast<uint64_t *>(sbeams)[tid] = beam_word;
+    if (tid < n1d + 4 * nm)
+      (&sk.S[0][0])[tid] = tid < n1d + 3 * nm ? const_word : iso_word;
+    __syncthreads();
+    if (mb) {
+      if (tid < ADM_MAX_BEAMS)
+        sbeams[tid].alpha =
+            member_alpha(sbeams[tid], gain, pmod, den, kc.log_01);
+      __syncthreads();
+    }
   }
+  if (first >= end) return;  // whole wavefronts
+  load_more(nat, nxt, more);
+  int sources_on = a.sources_on;
+  if (a.beam_table) {
+    sources_on = 0;
+    for (int b = 0; b < a.n_beams; ++b) sources_on |= sbeams[b].on ? 1 : 0;
+  }
+  // uniform constants, in scalar registers for the whole patch loop:
+  // in-plane shape values, collocation derivative, DcS, geometry and the
+  // kernel arguments the loop reads. For Q2 the host has checked that the
+  // middle Gauss point is the middle node (S row 1 = (0, 1, 0)), that S is
+  // symmetric under reflection except S[2][1] and that Dc is antisymmetric
+  // with Dc[1][1] = 0, bit for bit: S and Dc then take 8 scalar values
+  // instead of 18, and the middle rows' products by 0 and 1 are skipped,
+  // which leaves every sum as the generic chain gives it (x + 0 = x for the
+  // finite temperatures here).
+  double S[N][N], Dc[N][N], DS[N][N];
+  if constexpr (P == 2) {
+    const double s00 = in_sgpr(kc.S[0][0]), s01 = in_sgpr(kc.S[0][1]),
+                 s02 = in_sgpr(kc.S[0][2]), s21 = in_sgpr(kc.S[2][1]);
+    const double d00 = in_sgpr(kc.Dc[0][0]), d01 = in_sgpr(kc.Dc[0][1]),
+                 d02 = in_sgpr(kc.Dc[0][2]), d10 = in_sgpr(kc.Dc[1][0]);
+    S[0][0] = s00;
+    S[0][1] = s01;
+    S[0][2] = s02;
+    S[1][0] = -0.0;
+    S[1][1] = 1.0;
+    S[1][2] = 0.0;
+    S[2][0] = s02;
+    S[2][1] = s21;
+    S[2][2] = s00;
+    Dc[0][0] = d00;
+    Dc[0][1] = d01;
+    Dc[0][2] = d02;
+    Dc[1][0] = d10;
+    Dc[1][1] = 0.0;
+    Dc[1][2] = -d10;
+    Dc[2][0] = -d02;
+    Dc[2][1] = -d01;
+    Dc[2][2] = -d00;
+    const double e00 = in_sgpr(kc.DcS[0][0]), e01 = in_sgpr(kc.DcS[0][1]),
+                 e02 = in_sgpr(kc.DcS[0][2]), e10 = in_sgpr(kc.DcS[1][0]);
+    DS[0][0] = e00;
+    DS[0][1] = e01;
+    DS[0][2] = e02;
+    DS[1][0] = e10;
+    DS[1][1] = 0.0;
+    DS[1][2] = -e10;
+    DS[2][0] = -e02;
+    DS[2][1] = -e01;
+    DS[2][2] = -e00;
+  } else {
+#pragma unroll
+    for (int q = 0; q < N; ++q)
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        S[q][k] = in_sgpr(kc.S[q][k]);
+        Dc[q][k] = in_sgpr(kc.Dc[q][k]);
+        DS[q][k] = in_sgpr(kc.DcS[q][k]);
+      }
+  }
+  const double ihx2 = kc.inv_h2[0], ihy2 = kc.inv_h2[1],
+               ihz2 = kc.inv_h2[2];
+  // det w_x w_y of a point; w_z joins in the z integration. The 1-D weights
+  // are symmetric (checked on the host), so few of them differ.
+  double jxy[N][N];
+#pragma unroll
+  for (int qx = 0; qx < N; ++qx)
+#pragma unroll
+    for (int qy = 0; qy < N; ++qy) {
+      const int x = min(qx, N - 1 - qx), y = min(qy, N - 1 - qy);
+      jxy[qx][qy] = kc.jxy[min(x, y)][max(x, y)];
+    }
   double *const xb = lds + (PK == 2 ? n_mat * kPlaneMergedLds : 0) +
-                     wave * L::wave_lds;
+                     wave * a.plane_wave_lds;
   double *const myslot = xb + cw * L::cell_slots + s * SL;
   // slot of plane n of this lane's cell
   auto slot_of = [&](int n) { return xb + cw * L::cell_slots + n * SL; };
-  PatchLoad nxt;
-  load_patch(nxt);
+  // the lane's entries of the point arrays
+  double *const pa = xb + lane, *const pb = pa + L::points,
+               *const pc = pb + L::points;
   // the lane's place in a patch's block of the patch buffer
   const int64_t rowlen = (int64_t)npx * L::patch_nx;
   const int64_t E_lane =
       ((int64_t)s * npy * L::patch_ny + iy * P) * rowlen + ix * P;
   for (int r = first; r < end; r += stride) {
   wave_lds_sync();  // the previous patch's exchange reads are done
-  const int ppx = walk.px, ppy = ymajor ? walk.top : walk.mid,
-            ppz = ymajor ? walk.mid : walk.top;
+  const int ppx = nat.px, ppy = nat.py, ppz = nat.pz;
   const int cx = ppx * PX + ix, cy = ppy * PY + iy, cz = ppz;
   const bool in_mesh = cw < CPW && cx < lext0 && cy < lext1;
   const int64_t c = cx + (int64_t)nc0 * (cy + (int64_t)nc1 * cz);
@@ -515,22 +580,10 @@ __global__ void __launch_bounds__(256)
     }
   }
   const bool rotated = act && (meta & kRotated) != 0;
-  // the stored powder of the lane's points and the cell's direction, loaded
-  // ahead of the contractions
+  const double cs = more.cs, sn = more.sn;
   double pin[NS == 3 ? NP : 1];
-  if constexpr (NS == 3) {
 #pragma unroll
-    for (int q = 0; q < NP; ++q) pin[q] = 0.0;
-    if (pw) {
-#pragma unroll
-      for (int q = 0; q < NP; ++q) pin[q] = pw[q];
-    }
-  }
-  double cs = 1.0, sn = 0.0;
-  if (rotated) {
-    cs = cos_p[c];
-    sn = sin_p[c];
-  }
+  for (int q = 0; q < (NS == 3 ? NP : 1); ++q) pin[q] = more.pin[q];
 
   // ---- values: S along x, then y, in registers ---------------------------
   double v[NP];
@@ -551,8 +604,8 @@ __global__ void __launch_bounds__(256)
         t[qx + N * yy] = acc;
       }
     if (r + stride < end) {
-      walk.advance();
-      load_patch(nxt);
+      nat = PatchAt(by_npx, by_mid, ymajor, r + stride);
+      load_patch(nat, nxt);
     }
 #pragma unroll
     for (int qy = 0; qy < N; ++qy)
@@ -602,7 +655,14 @@ __global__ void __launch_bounds__(256)
 
   // ---- per-point physics, one point row (fixed y) at a time --------------
   bool near = false;
-  if (sources_on && act) {
+  // a patch outside the cells that a beam may reach skips the test of its
+  // cells (1,500 of a cold patch's 11,000 cycles)
+  const bool reach = sources_on && ppx * PX <= a.reach_hi[0] &&
+                     ppx * PX + PX > a.reach_lo[0] &&
+                     ppy * PY <= a.reach_hi[1] &&
+                     ppy * PY + PY > a.reach_lo[1] && ppz <= a.reach_hi[2] &&
+                     ppz >= a.reach_lo[2];
+  if (reach && act) {
     const int cc[3] = {cx, cy, cz};
     double lo[3], hi[3];
 #pragma unroll
@@ -768,9 +828,8 @@ __global__ void __launch_bounds__(256)
           k = sv * k + pv * __builtin_fma(d, kp1, kp0);
         }
         const double irc = recip(rho * cp);
-        // the source pass reads 1 / (rho c_p) from the lane's slot
-        myslot[q] = irc;
-        const double cq = ((-irc) * jxw[qx][qy]) * k;
+        pa[64 * q] = irc;  // for the source pass
+        const double cq = ((-irc) * jxy[qx][qy]) * k;
         w0[qx] = cq * (gxq * ax);
         w1[qx] = cq * (gyq * ay);
         w2[qx] = cq * (gz[q] * ihz2);
@@ -787,162 +846,196 @@ __global__ void __launch_bounds__(256)
     }
   };
 
-  // SOLID: the solid path (material mid_ for every lane, ratios (1, 0, 0));
-  // otherwise the lane's own material and the phase-state update
-  auto physics = [&](auto solid_tag, int mid_, const double *mB_,
-                     const double *mC_, const MergedBins &mbin_, bool iso_,
-                     bool rot_) {
+  // General form, in two steps. First the points' properties, a row at a
+  // time in a loop (the rows share one copy of the code, and the node-plane
+  // accumulators are not live yet: unrolled and in one step it spills), into
+  // the point arrays; then the fluxes and their folding, unrolled. The steps
+  // of a row run over its points together, so that their LDS reads overlap.
+  // SOLID: every point solid and material mid_ for every lane; otherwise the
+  // lane's own material and the phase-state update. OUT: 1/(rho c_p) and
+  // k_x (kIso), 1/(rho c_p) times the three conductivities (kAniso), or
+  // 1/(rho c_p) alone (kIrc).
+  constexpr int kIso = 0, kAniso = 1, kIrc = 2;
+  auto points = [&](auto solid_tag, auto out_tag, int mid_, const double *mB_,
+                    const double *mC_, const MergedBins &mbin_) {
     constexpr bool SOLID = decltype(solid_tag)::value;
+    constexpr int OUT = decltype(out_tag)::value;
     if constexpr (SOLID) solid_again();
-    // polynomial coefficients of the wave's solid material: uniform scalar
-    // loads, once per patch
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+      if constexpr (NS == 3 && !SOLID) pa[64 * q] = pin[q];
+      pb[64 * q] = Tq[q];
+    }
+    // polynomial coefficients of the wave's solid material: scalar loads
     const ADM_CONSTANT MatConst &mcst = kc.mat;
     constexpr bool POLY1 = PK == 0 && SOLID;
     const int order = POLY1 ? mcst.p_order : 0;
-    static_for<0, N>([&](auto qyc) {
-      constexpr int qy = decltype(qyc)::value;
-      double w0[N], w1[N], w2[N];
+#pragma unroll 1
+    for (int qy = 0; qy < N; ++qy) {
+      double *const ra = pa + 64 * N * qy, *const rb = pb + 64 * N * qy,
+                    *const rc = pc + 64 * N * qy;
       double Tr[N];
 #pragma unroll
-      for (int qx = 0; qx < N; ++qx) Tr[qx] = Tq[qx + N * qy];
+      for (int qx = 0; qx < N; ++qx) Tr[qx] = rb[64 * qx];
       int jr[N];
       if constexpr (PK == 2) merged_bin_intervals<N>(mB_, mbin_, Tr, jr);
-      // update_state_ratios (source/ThermalOperator.templates.hh:227-317):
-      // the mushy division where a point of the wavefront needs it
-      double mushy[N];
+      // update_state_ratios (source/ThermalOperator.templates.hh:227-317)
+      double r_[N][NS], l[N];
+#pragma unroll
+      for (int qx = 0; qx < N; ++qx) {
+        l[qx] = 0.0;
+        r_[qx][0] = 1.0;
+#pragma unroll
+        for (int k = 1; k < NS; ++k) r_[qx][k] = 0.0;
+      }
       if constexpr (!SOLID && NS > 1) {
+        // the mushy division where a point of the wavefront needs it
         bool need = false;
 #pragma unroll
         for (int qx = 0; qx < N; ++qx) {
-          mushy[qx] = 0.0;
+          l[qx] = Tr[qx] > liquidus ? 1.0 : 0.0;
           need |= !(Tr[qx] < solidus) && !(Tr[qx] > liquidus);
         }
         if (__any(need)) {
 #pragma unroll
-          for (int qx = 0; qx < N; ++qx)
-            mushy[qx] = (Tr[qx] - solidus) / (liquidus - solidus);
+          for (int qx = 0; qx < N; ++qx) {
+            const double mushy = (Tr[qx] - solidus) / (liquidus - solidus);
+            l[qx] = Tr[qx] < solidus ? 0.0
+                                     : (Tr[qx] > liquidus ? 1.0 : mushy);
+          }
+        }
+#pragma unroll
+        for (int qx = 0; qx < N; ++qx) {
+          const int q = qx + N * qy;
+          if constexpr (NS == 2) {
+            r_[qx][1] = l[qx];
+            r_[qx][0] = 1.0 - l[qx];
+          } else {
+            const double p0 = ra[64 * qx];
+            const double am = 1.0 - l[qx];
+            const double pv = (p0 < am) ? p0 : am;
+            r_[qx][1] = l[qx];
+            r_[qx][2] = pv;
+            r_[qx][0] = 1.0 - l[qx] - pv;
+            if (pw && pv != p0) pw[q] = pv;
+          }
+          if (lq && (l[qx] != 0.0 || dirty)) lq[q] = l[qx];
+          plane_liquid |= l[qx] != 0.0;
         }
       }
-      double rho_[N], cp_[N], kx_[N], ky_[N], kz_[N];
+      // get_inv_rho_cp (source/ThermalOperator.templates.hh:415-477) and the
+      // conductivities
+      double rho[N], cp[N], kx[N], ky[N], kzz[N];
       if constexpr (POLY1) {
         // sum_i c_i T^i, state ratio 1
         double tp[N];
 #pragma unroll
         for (int qx = 0; qx < N; ++qx) {
           tp[qx] = 1.0;
-          rho_[qx] = cp_[qx] = kx_[qx] = ky_[qx] = kz_[qx] = 0.0;
+          rho[qx] = cp[qx] = kx[qx] = ky[qx] = kzz[qx] = 0.0;
         }
 #pragma unroll
         for (int i = 0; i < ADM_MAX_POLY; ++i) {
           if (i > order) break;
-          const double cr = mcst.poly[mid_][ADM_DENSITY][0][i];
-          const double cc = mcst.poly[mid_][ADM_SPECIFIC_HEAT][0][i];
-          const double ck =
-              mcst.poly[mid_][ADM_THERMAL_CONDUCTIVITY_X][0][i];
-          const double cy_ =
-              mcst.poly[mid_][ADM_THERMAL_CONDUCTIVITY_Y][0][i];
-          const double cz_ =
-              mcst.poly[mid_][ADM_THERMAL_CONDUCTIVITY_Z][0][i];
+          const auto &pcf = mcst.poly[mid_];
 #pragma unroll
           for (int qx = 0; qx < N; ++qx) {
             if (i > 0) tp[qx] = tp[qx] * Tr[qx];
-            rho_[qx] += cr * tp[qx];
-            cp_[qx] += cc * tp[qx];
-            kx_[qx] += ck * tp[qx];
-            ky_[qx] += cy_ * tp[qx];
-            kz_[qx] += cz_ * tp[qx];
+            rho[qx] += pcf[ADM_DENSITY][0][i] * tp[qx];
+            cp[qx] += pcf[ADM_SPECIFIC_HEAT][0][i] * tp[qx];
+            if constexpr (OUT != kIrc)
+              kx[qx] += pcf[ADM_THERMAL_CONDUCTIVITY_X][0][i] * tp[qx];
+            if constexpr (OUT == kAniso) {
+              ky[qx] += pcf[ADM_THERMAL_CONDUCTIVITY_Y][0][i] * tp[qx];
+              kzz[qx] += pcf[ADM_THERMAL_CONDUCTIVITY_Z][0][i] * tp[qx];
+            }
           }
         }
-      }
-#pragma unroll
-      for (int qx = 0; qx < N; ++qx) {
-        const int q = qx + N * qy;
-        const double T = Tr[qx];
-        double gxq, gyq;
-        grad_xy(qx, qy, gxq, gyq);
-        double r_[NS];
-        double l = 0.0;
-        if constexpr (SOLID || NS == 1) {
-          r_[0] = 1.0;
-#pragma unroll
-          for (int k = 1; k < NS; ++k) r_[k] = 0.0;
-        } else {
-          double p0 = 0.0;
-          if constexpr (NS == 3) p0 = pin[q];
-          double pv = p0;
-          l = T < solidus ? 0.0 : (T > liquidus ? 1.0 : mushy[qx]);
-          if constexpr (NS == 2) {
-            r_[1] = l;
-            r_[0] = 1.0 - l;
-          } else {
-            const double am = 1.0 - l;
-            pv = (pv < am) ? pv : am;
-            r_[1] = l;
-            r_[2] = pv;
-            r_[0] = 1.0 - l - pv;
-          }
-          if (pw && pv != p0) pw[q] = pv;
-          if (lq && (l != 0.0 || dirty)) lq[q] = l;
-          plane_liquid |= l != 0.0;
-        }
-        double irc, kx, ky, kzz;
-        auto props = [&](const auto &ev) {
-          // get_inv_rho_cp (source/ThermalOperator.templates.hh:415-477)
-          const double density = ev(ADM_DENSITY, r_);
-          double specific_heat = ev(ADM_SPECIFIC_HEAT, r_);
-          if constexpr (NS > 1 && !SOLID) {
-            const double is_mushy = r_[1] * r_[0];
-            if (is_mushy > 0.0) specific_heat += latent;
-          }
-          irc = recip(density * specific_heat);
-          kx = ev(ADM_THERMAL_CONDUCTIVITY_X, r_);
-          if (iso_) {
-            ky = kx;
-            kzz = kx;
-          } else {
-            ky = ev(ADM_THERMAL_CONDUCTIVITY_Y, r_);
-            kzz = ev(ADM_THERMAL_CONDUCTIVITY_Z, r_);
+      } else {
+        auto props = [&](const auto &ev, int qx) {
+          rho[qx] = ev(ADM_DENSITY, r_[qx]);
+          cp[qx] = ev(ADM_SPECIFIC_HEAT, r_[qx]);
+          if constexpr (OUT != kIrc)
+            kx[qx] = ev(ADM_THERMAL_CONDUCTIVITY_X, r_[qx]);
+          if constexpr (OUT == kAniso) {
+            ky[qx] = ev(ADM_THERMAL_CONDUCTIVITY_Y, r_[qx]);
+            kzz[qx] = ev(ADM_THERMAL_CONDUCTIVITY_Z, r_[qx]);
           }
         };
-        if constexpr (POLY1) {
-          irc = recip(rho_[qx] * cp_[qx]);
-          kx = kx_[qx];
-          ky = ky_[qx];
-          kzz = kz_[qx];
-        } else if constexpr (PK == 2) {
-          const int j = jr[qx];
-          if constexpr (SOLID) {
+#pragma unroll
+        for (int qx = 0; qx < N; ++qx) {
+          if constexpr (PK == 2 && SOLID) {
             // the solid value alone: (0 + 1 X_s) + 0 X_l + 0 X_p = X_s
-            const double d = T - mB_[j > 0 ? j - 1 : 0];
+            const int j = jr[qx];
+            const double d = Tr[qx] - mB_[j > 0 ? j - 1 : 0];
             const double *cj = mC_ + j * (ADM_MAX_STATES * 2);
             auto solid_ev = [&](int prop, const double(&)[NS]) {
               const double *cf = cj + prop * (kMergedMax * ADM_MAX_STATES * 2);
               return __builtin_fma(d, cf[1], cf[0]);
             };
-            props(solid_ev);
+            props(solid_ev, qx);
+          } else if constexpr (PK == 2) {
+            props(MergedEval(mB_, mC_, Tr[qx], jr[qx]), qx);
           } else {
-            props(MergedEval(mB_, mC_, T, j));
+            props(typename EvalOf<PK>::type(m, mid_, Tr[qx]), qx);
+          }
+        }
+      }
+#pragma unroll
+      for (int qx = 0; qx < N; ++qx) {
+        double c_p = cp[qx];
+        if constexpr (!SOLID && NS > 1) {
+          const double is_mushy = r_[qx][1] * r_[qx][0];
+          if (is_mushy > 0.0) c_p += latent;
+        }
+        const double irc = recip(rho[qx] * c_p);
+        ra[64 * qx] = OUT == kAniso ? irc * kx[qx] : irc;
+        if constexpr (OUT == kIso) rb[64 * qx] = kx[qx];
+        if constexpr (OUT == kAniso) {
+          rb[64 * qx] = irc * ky[qx];
+          rc[64 * qx] = irc * kzz[qx];
+        }
+      }
+    }
+  };
+  // -(1/rho c_p) K grad T * JxW, each component with its 1/h, from the point
+  // arrays
+  auto fluxes = [&](auto iso_tag) {
+    constexpr bool ISO = decltype(iso_tag)::value;
+    // isotropic cells: the lanes that take the rotated form
+    const bool turned = ISO && (fast ? __any(rotated) != 0 : rotated);
+    const bool any_turned = __any(turned);
+    const double ihxy = kc.inv_h[0] * kc.inv_h[1];
+    static_for<0, N>([&](auto qyc) {
+      constexpr int qy = decltype(qyc)::value;
+      double w0[N], w1[N], w2[N];
+#pragma unroll
+      for (int qx = 0; qx < N; ++qx) {
+        const int q = qx + N * qy;
+        double gxq, gyq;
+        grad_xy(qx, qy, gxq, gyq);
+        if constexpr (ISO) {
+          const double cq = (-pa[64 * q]) * jxy[qx][qy], k = pb[64 * q];
+          w0[qx] = (cq * k) * (gxq * ihx2);
+          w1[qx] = (cq * k) * (gyq * ihy2);
+          w2[qx] = (cq * k) * (gz[q] * ihz2);
+          if (any_turned) {
+            const double ih0 = kc.inv_h[0], ih1 = kc.inv_h[1];
+            const double fx = (k * cs * cs + k * sn * sn) * (gxq * ih0);
+            const double fy = (k * sn * sn + k * cs * cs) * (gyq * ih1);
+            w0[qx] = turned ? (cq * fx) * ih0 : w0[qx];
+            w1[qx] = turned ? (cq * fy) * ih1 : w1[qx];
           }
         } else {
-          props(typename EvalOf<PK>::type(m, mid_, T));
+          const double c0 = (-pa[64 * q]) * jxy[qx][qy];
+          const double c1 = (-pb[64 * q]) * jxy[qx][qy];
+          const double c2 = (-pc[64 * q]) * jxy[qx][qy];
+          // (c0, c1) rotated into the deposition direction
+          const double cxy = ((c0 - c1) * sn * cs) * ihxy;
+          w0[qx] = (c0 * cs * cs + c1 * sn * sn) * (gxq * ihx2) + cxy * gyq;
+          w1[qx] = cxy * gxq + (c0 * sn * sn + c1 * cs * cs) * (gyq * ihy2);
+          w2[qx] = c2 * (gz[q] * ihz2);
         }
-        myslot[q] = irc;  // for the source pass
-        // -(1/rho c_p) K grad T * JxW, each component with its 1/h
-        const double cq = (-irc) * jxw[qx][qy];
-        if (rot_) {
-          const double ih0 = kc.inv_h[0], ih1 = kc.inv_h[1];
-          const double gx_ = gxq * ih0, gy_ = gyq * ih1;
-          const double fx = (kx * cs * cs + ky * sn * sn) * gx_ +
-                            ((kx - ky) * sn * cs) * gy_;
-          const double fy = ((kx - ky) * sn * cs) * gx_ +
-                            (kx * sn * sn + ky * cs * cs) * gy_;
-          w0[qx] = (cq * fx) * ih0;
-          w1[qx] = (cq * fy) * ih1;
-        } else {
-          w0[qx] = (cq * kx) * (gxq * ihx2);
-          w1[qx] = (cq * ky) * (gyq * ihy2);
-        }
-        w2[qx] = (cq * kzz) * (gz[q] * ihz2);
       }
       fold_row(qy, w0, w1, w2);
     });
@@ -952,34 +1045,50 @@ __global__ void __launch_bounds__(256)
       one_interval(std::integral_constant<bool, NS == 3>{});
     else
       one_interval(std::integral_constant<bool, false>{});
-  } else if (fast) {
+  } else {
+    constexpr std::integral_constant<bool, true> yes{};
+    constexpr std::integral_constant<bool, false> no{};
+    constexpr std::integral_constant<int, kIso> iso_out{};
+    constexpr std::integral_constant<int, kAniso> aniso_out{};
     // the wave's material (uniform: scalar registers, uniform LDS rows)
     const double *fB = lds + mid0 * kPlaneMergedLds;
-    physics(std::integral_constant<bool, true>{}, mid0, fB, fB + kMergedMax,
-            *reinterpret_cast<const MergedBins *>(fB + kMergedLds),
-            __builtin_amdgcn_readfirstlane(sk.iso[mid0] != 0.0 ? 1 : 0) != 0,
-            __any(rotated));
-  } else {
-    physics(std::integral_constant<bool, false>{}, mid, mB, mC, mbin, iso,
-            rotated);
+    const MergedBins &fbin =
+        *reinterpret_cast<const MergedBins *>(fB + kMergedLds);
+    if (!__any(act && !iso)) {
+      if (fast)
+        points(yes, iso_out, mid0, fB, fB + kMergedMax, fbin);
+      else
+        points(no, iso_out, mid, mB, mC, mbin);
+      fluxes(yes);
+    } else {
+      if (fast)
+        points(yes, aniso_out, mid0, fB, fB + kMergedMax, fbin);
+      else
+        points(no, aniso_out, mid, mB, mC, mbin);
+      fluxes(no);
+      // the source pass needs 1/(rho c_p) alone (the state update again
+      // changes nothing)
+      if (reach && __any(near))
+        points(no, std::integral_constant<int, kIrc>{}, mid, mB, mC, mbin);
+    }
   }
   // heat sources, in a pass of their own over the cells that a beam can
-  // reach (few), a point row at a time: 1/(rho c_p) as the physics left it
-  // in the lane's slot, then Ap[xx, yy] += S[qy][yy] (S^T val)[xx]
-  if (__any(near)) {
+  // reach (few), a point row at a time: 1/(rho c_p) from the point
+  // array, then Ap[xx, yy] += S[qy][yy] (S^T val)[xx]
+  if (reach && __any(near)) {
     wave_lds_sync();
     if (near) {
-      plane_source<P>((ADM_LDS double *)myslot,
+      plane_source<P>((ADM_LDS double *)pa,
                       (const ADM_LDS adm_beam_state *)&sbeams[0], a.n_beams,
                       (const ADM_LDS CellConstLds *)&sk, &kc, cx, cy, cz, s);
 #pragma unroll
       for (int qy = 0; qy < N; ++qy)
 #pragma unroll
         for (int xx = 0; xx < N; ++xx) {
-          double tv = S[0][xx] * myslot[N * qy];
+          double tv = S[0][xx] * pa[64 * N * qy];
 #pragma unroll
           for (int q = 1; q < N; ++q)
-            tv = __builtin_fma(S[q][xx], myslot[q + N * qy], tv);
+            tv = __builtin_fma(S[q][xx], pa[64 * (q + N * qy)], tv);
 #pragma unroll
           for (int yy = 0; yy < N; ++yy)
             Ap[xx + N * yy] = __builtin_fma(S[qy][yy], tv, Ap[xx + N * yy]);
@@ -994,8 +1103,8 @@ __global__ void __launch_bounds__(256)
   }
 
   // ---- exchange 2: z part, node plane s = sum over point planes ----------
-  // out = sum_qz S[qz][s] Ap_qz + sum_qz (Dc S)[qz][s] Bp_qz, the two
-  // parts in a buffer each
+  // out = sum_qz w_qz (S[qz][s] Ap_qz + (Dc S)[qz][s] Bp_qz), the two parts
+  // in a buffer each
   double out[NP];
   wave_lds_sync();
 #pragma unroll
@@ -1008,8 +1117,8 @@ __global__ void __launch_bounds__(256)
     double sc[N], dc[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      sc[k] = sk.S[k][s];
-      dc[k] = sk.Dc[k][s];  // (Dc S)[k][s]
+      sc[k] = sk.S[k][s] * sk.wq[k];
+      dc[k] = sk.Dc[k][s] * sk.wq[k];  // (Dc S)[k][s]
     }
 #pragma unroll
     for (int q = 0; q < NP; ++q) out[q] = sc[0] * slot_of(0)[q];
@@ -1047,6 +1156,7 @@ __global__ void __launch_bounds__(256)
   // their wait from including the stores below
 #pragma unroll
   for (int q = 0; q < NP; ++q) asm volatile("" : "+v"(nxt.u[q]));
+  if (r + stride < end) load_more(nat, nxt, more);
   if (in_mesh) {
   // the patch's node sums, every node of the patch once, into its slots
   // of the patch buffer (plain stores; the gather kernel adds the slots of
