@@ -1,0 +1,54 @@
+"""The localised EnKF update at the edges of its matrix tiles (16 members,
+16 observations, 16 nodes), and with an observation that is not finite."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def setup(N, m, seed):
+    from tests.test_gpu_enkf import ensemble
+    base, ens = ensemble(N)
+    rng = np.random.RandomState(seed)
+    X = 1000.0 + rng.normal(scale=30.0, size=(N, ens.n_dofs))
+    obs = np.sort(rng.permutation(ens.n_dofs)[:m]).astype(np.int64)
+    y = 1000.0 + rng.normal(scale=5.0, size=m)
+    R = np.diag(rng.uniform(1.0, 4.0, m))
+    return base, ens, X, obs, y, R, rng.normal(0.0, 1.5, (N, m))
+
+
+def update(ens, base, fn, cutoff, X, obs, y, R, noise):
+    import torch
+    from adamantine_amd.ensemble import DataAssimilator
+    da = DataAssimilator(fn, cutoff)
+    da.update_dof_mapping(ens, base.node_coordinates()[obs])
+    dev = torch.tensor(X, device="cuda")
+    da.update_ensemble(ens, dev, y, R, noise=noise)
+    return dev.cpu().numpy()
+
+
+@pytest.mark.parametrize("fn", ["step_function", "gaspari_cohn"])
+@pytest.mark.parametrize("N,m", [(2, 1), (15, 16), (16, 17), (17, 15),
+                                 (33, 31), (48, 33), (49, 20), (64, 40)])
+def test_localized_update_edges(N, m, fn):
+    from adamantine_amd.ensemble import LOCALIZATION
+    from tests.test_gpu_enkf import oracle_analysis
+    base, ens, X, obs, y, R, noise = setup(N, m, 7 * N + m)
+    got = update(ens, base, fn, 0.9e-3, X, obs, y, R, noise)
+    want, _ = oracle_analysis(base, X.copy(), None, obs, y, R, noise,
+                              LOCALIZATION[fn], 0.9e-3)
+    scale = np.abs(want - X).max()
+    # the bar of test_gpu_enkf: solves of two precisions
+    assert np.abs(got - want).max() <= 1e-10 * scale + 1e-12 * 1000
+
+
+def test_localized_update_not_finite():
+    """Nodes out of the observation's reach keep their values."""
+    base, ens, X, obs, y, R, noise = setup(5, 1, 3)
+    y[0] = np.inf
+    got = update(ens, base, "gaspari_cohn", 0.6e-3, X, obs, y, R, noise)
+    xyz = base.node_coordinates()
+    far = np.linalg.norm(xyz - xyz[obs[0]], axis=1) > 0.6e-3
+    assert far.any() and not far.all()
+    np.testing.assert_allclose(got[:, far], X[:, far], rtol=1e-14)
+    assert not np.isfinite(got[:, obs[0]]).any()
