@@ -418,7 +418,7 @@ Context::Context(const adm_problem_desc &d) {
     use_coloring = !(e[0] == '1');
   {
     const char *e = std::getenv("ADM_CELL_KERNEL");
-    use_plane = d.mesh.fe_degree <= 2 && !(e && std::string(e) == "line");
+    use_plane = d.mesh.fe_degree <= kPlaneMaxDegree && !(e && std::string(e) == "line");
   }
   if (const char *e = std::getenv("ADM_XCD_ORDER")) xcd_order = e[0] == '1';
   {
@@ -504,6 +504,12 @@ Context::Context(const adm_problem_desc &d) {
       for (int k = 0; k < n1; ++k)
         acc += (long double)kc.Dc[q][k] * (long double)kc.S[k][i];
       kc.DcS[q][i] = (double)acc;
+    }
+  for (int q = 0; q < n1; ++q)
+    for (int i = 0; i < n1; ++i) {
+      const int qr = n1 - 1 - q, ir = n1 - 1 - i;
+      kc.aDc[q][i] = 0.5 * (kc.Dc[q][i] - kc.Dc[qr][ir]);
+      kc.aDcS[q][i] = 0.5 * (kc.DcS[q][i] - kc.DcS[qr][ir]);
     }
   // the plane kernel's Q2 form relies on these equalities of the 1-D
   // tables (they hold for the Gauss and Gauss-Lobatto rules); without them
@@ -1272,12 +1278,28 @@ void Context::apply(const double *src, double *dst, int add, hipStream_t s,
   launch(a, face_args(), src, dst, 1, s, nz_active, patch);
 }
 
+// the plane kernel's patch shape and LDS for FE degree p
+struct PlaneShape {
+  int px, py, wave_lds, wave_lds_aniso;
+  int64_t patch_nodes;
+};
+template <int P>
+static PlaneShape plane_shape_of() {
+  using L = PlaneLanes<P>;
+  return {L::PX, L::PY, L::wave_lds, L::wave_lds_aniso, L::patch_nodes};
+}
+static PlaneShape plane_shape(int p) {
+  return p == 1   ? plane_shape_of<1>()
+         : p == 2 ? plane_shape_of<2>()
+                  : plane_shape_of<3>();
+}
+
 // Cell and face kernels of the context's configuration; with n_members > 1
 // the arguments carry the member table and the grid's y index is the member.
 void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
                      double *dst, unsigned n_members, hipStream_t s,
                      int nz_rows, double *patch, const StageArgs *st) const {
-  if (st && !(use_plane && p <= 2))
+  if (st && !plane_path())
     throw AdmError(ADM_ERR_INVALID, "a fused stage needs the plane kernel");
   StageArgs stage;
   std::memset(&stage, 0, sizeof(stage));
@@ -1322,7 +1344,7 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
     ADM_DISPATCH(5, 3)
 #undef ADM_DISPATCH
   };
-  const bool plane = use_plane && p <= 2;
+  const bool plane = plane_path();
   if (plane) {
     // one launch, one PX x PY cell patch of a cell layer per wavefront
     const size_t plds =
@@ -1330,13 +1352,12 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
     CellArgs ac = a;
     ac.color = -1;
     for (int d = 0; d < 3; ++d) ac.lext[d] = lim[d];
-    const int px = p == 1 ? PlaneLanes<1>::PX : PlaneLanes<2>::PX;
-    const int py = p == 1 ? PlaneLanes<1>::PY : PlaneLanes<2>::PY;
+    const PlaneShape shape = plane_shape(p);
+    const int px = shape.px, py = shape.py;
     ac.plane_npx = (lim[0] + px - 1) / px;
     ac.plane_npy = (lim[1] + py - 1) / py;
     ac.n_rows = ac.plane_npx * ac.plane_npy * lim[2];
-    const int64_t slots = p == 1 ? PlaneLanes<1>::patch_nodes
-                                 : PlaneLanes<2>::patch_nodes;
+    const int64_t slots = shape.patch_nodes;
     if (ac.beam_table) {
       // the beams of a captured loop are not known here
       for (int d = 0; d < 3; ++d) {
@@ -1347,11 +1368,8 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
       beam_reach(ac.beams, ac.n_beams, kc.origin, kc.inv_h, ac.reach_lo,
                  ac.reach_hi);
     }
-    const bool iso = all_isotropic();
-    ac.plane_wave_lds = p == 1 ? (iso ? PlaneLanes<1>::wave_lds
-                                      : PlaneLanes<1>::wave_lds_aniso)
-                               : (iso ? PlaneLanes<2>::wave_lds
-                                      : PlaneLanes<2>::wave_lds_aniso);
+    ac.plane_wave_lds =
+        all_isotropic() ? shape.wave_lds : shape.wave_lds_aniso;
     ac.plane_E_stride = (int64_t)ac.n_rows * slots;
     if (patch) {
       if ((size_t)ac.plane_E_stride * M > kNoAllocScratchDoubles)
@@ -1365,12 +1383,15 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
       ac.plane_E = ensure_patch_buffer((size_t)ac.plane_E_stride * M);
     }
     if (ac.n_rows > 0) {
-      // a persistent grid: as many blocks as the chip holds at the
-      // kernel's occupancy (shared among the members), each looping over
-      // patches; at least 8 blocks, one per XCD
+      // a persistent grid: 2 wavefronts per SIMD, as many blocks as the
+      // chip holds at the occupancy of Q1 and Q2 (shared among the
+      // members), each looping over patches; at least 8 blocks, one per
+      // XCD. Q3 holds half of them at a time: the other half, started as
+      // blocks end, evens out the uneven patches (193 us per RK4 step of
+      // 50x25x17 cells against 206 with one grid of resident blocks)
       const int64_t full = (ac.n_rows + cell_waves - 1) / cell_waves;
       const int64_t resident =
-          (int64_t)n_cu * 4 * kPlaneWavesPerEU / cell_waves / (int64_t)M;
+          (int64_t)n_cu * 4 * 2 / cell_waves / (int64_t)M;
       const int64_t nb = std::min(full, std::max<int64_t>(8, resident));
 #define ADM_DISPATCH(P_, NS_)                                              \
   if (p == P_ && n_states == NS_) {                                         \
@@ -1387,6 +1408,9 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
       ADM_DISPATCH(2, 1)
       ADM_DISPATCH(2, 2)
       ADM_DISPATCH(2, 3)
+      ADM_DISPATCH(3, 1)
+      ADM_DISPATCH(3, 2)
+      ADM_DISPATCH(3, 3)
 #undef ADM_DISPATCH
     }
     // the face term's slots, then the second pass: every node's sum from
@@ -1402,22 +1426,18 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
                                                      (int64_t)p * lim[2] + 1))
            : n_dofs;
     const dim3 ggrid((unsigned)((n_gather + 255) / 256), M);
-    if (p == 1)
-      hipLaunchKernelGGL(plane_gather_kernel<1>, ggrid, dim3(256), 0, s,
-                         ac.plane_E, ac.plane_E_stride, dst,
-                         a.members ? a.member_stride : (int64_t)0, nn[0],
-                         nn[1], nn[2], ac.plane_npx, ac.plane_npy, lim[2],
-                         a.add, fa, stage);
-    else
-      hipLaunchKernelGGL(plane_gather_kernel<2>, ggrid, dim3(256), 0, s,
-                         ac.plane_E, ac.plane_E_stride, dst,
-                         a.members ? a.member_stride : (int64_t)0, nn[0],
-                         nn[1], nn[2], ac.plane_npx, ac.plane_npy, lim[2],
-                         a.add, fa, stage);
+    const auto gather = p == 1   ? plane_gather_kernel<1>
+                        : p == 2 ? plane_gather_kernel<2>
+                                 : plane_gather_kernel<3>;
+    hipLaunchKernelGGL(gather, ggrid, dim3(256), 0, s, ac.plane_E,
+                       ac.plane_E_stride, dst,
+                       a.members ? a.member_stride : (int64_t)0, nn[0], nn[1],
+                       nn[2], ac.plane_npx, ac.plane_npy, lim[2], a.add, fa,
+                       stage);
   }
   // the line kernel runs once per parity color (cells of one color share no
   // node: plain read-add-write of dst), or once with atomics
-  const int n_colors = (use_plane && p <= 2) ? 0 : (use_coloring ? 8 : 1);
+  const int n_colors = plane ? 0 : (use_coloring ? 8 : 1);
   const int cpw = cells_per_wave(p);
   for (int col = 0; col < n_colors; ++col) {
     CellArgs ac = a;
@@ -1557,12 +1577,10 @@ void Context::launch_2d(const CellArgs &a, const FaceArgs &fa,
 
 size_t Context::patch_buffer_size(int nz_rows, unsigned n_members) const {
   const int nz = nz_rows >= 0 ? std::min(nz_rows, nc[2]) : nc[2];
-  const int px = p == 1 ? PlaneLanes<1>::PX : PlaneLanes<2>::PX;
-  const int py = p == 1 ? PlaneLanes<1>::PY : PlaneLanes<2>::PY;
-  const size_t slots =
-      p == 1 ? PlaneLanes<1>::patch_nodes : PlaneLanes<2>::patch_nodes;
-  return (size_t)((nc[0] + px - 1) / px) * ((nc[1] + py - 1) / py) * nz *
-         slots * n_members;
+  const PlaneShape shape = plane_shape(p);
+  return (size_t)((nc[0] + shape.px - 1) / shape.px) *
+         ((nc[1] + shape.py - 1) / shape.py) * nz * shape.patch_nodes *
+         n_members;
 }
 
 double *Context::ensure_patch_buffer(size_t n) const {
@@ -1922,6 +1940,7 @@ Ensemble::Ensemble(const adm_problem_desc &base, int n,
   n_dofs = members[0]->n_dofs;
   auto work = std::make_shared<ActWork>();
   for (auto &m : members) m->act = work;
+  members[0]->reserve_patch_buffer(n);
   refresh_members();
 }
 
@@ -2241,7 +2260,9 @@ extern "C" {
 int adm_create(const adm_problem_desc *desc, void **out) {
   ADM_API_BEGIN
   if (!desc || !out) return adm::set_error(ADM_ERR_INVALID, "null argument");
-  *out = new Context(*desc);
+  auto ctx = std::make_unique<Context>(*desc);
+  ctx->reserve_patch_buffer(1);
+  *out = ctx.release();
   ADM_API_END
 }
 
@@ -2362,7 +2383,17 @@ int adm_vmult_noalloc(void *ptr, const double *src, double *dst, int add,
   ADM_CTX(ptr)
   if (!src || !dst) return adm::set_error(ADM_ERR_INVALID, "null vector");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // as adm_vmult, with the scratch array as the patch buffer
+  // as adm_vmult, with the scratch array as the patch buffer; Q3, whose patch
+  // buffer is larger than the array for meshes that this call takes, through
+  // the line kernel
+  struct Line {
+    adm::Context &c;
+    const bool plane;
+    explicit Line(adm::Context &c_) : c(c_), plane(c_.use_plane) {
+      if (c.p == 3) c.use_plane = false;
+    }
+    ~Line() { c.use_plane = plane; }
+  } line(ctx);
   if (ctx.n_ext >= 0) {
     ctx.to_nodes(src, ctx.d_map_src, s);
     if (!ctx.plane_path()) ctx.fill(ctx.d_map_dst, 0.0, ctx.n_dofs, s);
@@ -2432,7 +2463,7 @@ static void tune_launch(adm::Context &cfg,
     for (int w = 2; w <= 4; ++w, ++k) {
       const int mode = modes[mi];
       if (mode == ADM_LAUNCH_PLANE &&
-          (cfg.p > 2 || cfg.n_dofs >= (int64_t)INT32_MAX ||
+          (cfg.p > kPlaneMaxDegree || cfg.n_dofs >= (int64_t)INT32_MAX ||
            !cfg.plane_tables_ok || cfg.dim == 2)) {
         if (ms_out) ms_out[k] = -1.0;
         continue;

@@ -3,7 +3,7 @@
 #include "adm_kernels.hpp"
 #include "adm_kernels_2d.hpp"
 #include "adm_launch.hpp"
-#if ADM_P <= 2
+#if ADM_P <= 3
 #include "adm_plane_kernel.hpp"
 #endif
 
@@ -20,7 +20,7 @@ void launch_cell(const CellArgs &a, const double *src, double *dst,
                      dim3(64 * waves), lds_bytes + xbytes, s, a, src, dst);
 }
 
-#if ADM_P <= 2
+#if ADM_P <= 3
 template <int P, int NS, int PK>
 void launch_plane(const CellArgs &a, const double *src, double *dst,
                   int64_t n_blocks, size_t lds_bytes, unsigned n_members,

@@ -99,6 +99,9 @@ struct GeomSnap {
   ~GeomSnap();
 };
 
+// FE degrees that the plane kernel covers
+constexpr int kPlaneMaxDegree = 3;
+
 struct Context {
   explicit Context(const adm_problem_desc &d);
   ~Context();
@@ -180,7 +183,13 @@ struct Context {
   // doubles of the patch buffer for launches over nz_rows cell layers
   size_t patch_buffer_size(int nz_rows, unsigned n_members) const;
   // the cell term goes through the plane kernel (which writes every node)
-  bool plane_path() const { return use_plane && p <= 2; }
+  bool plane_path() const { return use_plane && p <= kPlaneMaxDegree; }
+  // Q3: the patch buffer of every cell layer, when the operator is created
+  // (its vmult allocates nothing later, also not while a stream is captured)
+  void reserve_patch_buffer(unsigned n_members) const {
+    if (p == 3 && plane_path())
+      ensure_patch_buffer(patch_buffer_size(-1, n_members));
+  }
   void compute_inverse_mass(double *out, hipStream_t s);
   void ensure_step_buffers(int method);
   void step(int method, double t, double dt, double *T, hipStream_t s);
@@ -244,7 +253,7 @@ struct Context {
   // line kernel: 8 parity colors without atomics, or one atomic launch
   // (ADM_CELL_ATOMICS=1 in the environment at creation)
   bool use_coloring = true;
-  // plane kernel (FE degrees 1 and 2; the default there unless
+  // plane kernel (FE degrees 1 to 3; the default there unless
   // ADM_CELL_KERNEL=line is in the environment at creation)
   bool use_plane = false;
   // the 1-D tables have the symmetries the plane kernel's Q2 form uses

@@ -82,6 +82,9 @@ struct KConst {
   double S[kMaxN][kMaxN];    // shape values  S[q][i] = l_i(x_q)
   double Dc[kMaxN][kMaxN];   // collocation derivative at the quadrature points
   double DcS[kMaxN][kMaxN];  // Dc * S: derivative at the points from nodes
+  // Dc and Dc S with M[n-1-q][n-1-i] = -M[q][i] to the last bit (the mean of
+  // the two entries)
+  double aDc[kMaxN][kMaxN], aDcS[kMaxN][kMaxN];
   double xq[kMaxN];
   double wq[kMaxN];          // 1-D quadrature weights
   double det;                // cell Jacobian determinant

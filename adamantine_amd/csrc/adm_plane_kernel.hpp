@@ -1,4 +1,4 @@
-// Plane cell kernel of the matrix-free heat operator for FE degrees 1 and 2
+// Plane cell kernel of the matrix-free heat operator for FE degrees 1 to 3
 // (gfx950). Reference: source/ThermalOperator.templates.hh:479-617.
 //
 // Lane layout: p+1 lanes per cell, lane s owning the x-y plane z = s of the
@@ -7,8 +7,8 @@
 // registers; only the z direction crosses lanes, through a wave-private LDS
 // buffer: one exchange for the evaluation and one for the integration
 // (against six in the line-per-lane kernel). A wavefront takes a patch of
-// PX x PY cells of one cell layer (7 x 3 for Q2: 63 lanes; 8 x 4 for Q1:
-// 64 lanes), so the nodes its cells share along x and y are summed inside
+// PX x PY cells of one cell layer (7 x 3 for Q2: 63 lanes; 8 x 4 for Q1 and
+// 4 x 4 for Q3: 64 lanes), so the nodes its cells share along x and y are summed inside
 // the wavefront (cross-lane shuffles). Each patch then stores its node sums
 // in its own block of a patch buffer, and a second kernel (one lane per
 // node) adds the blocks of the patches that share the node, in a fixed
@@ -47,7 +47,8 @@
 //  - the two parts of the integration share one exchange.
 // 128x64x32 Q2, per application (plane + gather + face kernels): 100.4 us
 // before, 76.9 us with these; 64 members of 64x32x16, per RK4 step: 3.17 ms
-// before, 2.39 ms; Q1 101x67x33: 38.6 us before, 28.6 us. What is left of the
+// before, 2.39 ms; Q1 101x67x33: 38.6 us before, 28.6 us. Q3 (line kernel in
+// 8 colour launches before), RK4 step of 50x25x17: 433 us before, 193 us. What is left of the
 // large launch is its slowest wavefront (melt under the beam: 133,000 cycles
 // against a mean of 87,000). Handing patches out by a counter instead of a
 // fixed share took 73 us there, but the counter's round trip cost the short
@@ -66,16 +67,18 @@ namespace adm {
 
 template <int P>
 struct PlaneLanes {
-  static_assert(P == 1 || P == 2, "plane kernel: FE degree 1 or 2");
+  static_assert(P >= 1 && P <= 3, "plane kernel: FE degrees 1 to 3");
   static constexpr int N = P + 1;
   static constexpr int NP = N * N;  // values per lane
-  static constexpr int PX = P == 1 ? 8 : 7;
-  static constexpr int PY = P == 1 ? 4 : 3;
+  static constexpr int PX = P == 1 ? 8 : (P == 2 ? 7 : 4);
+  static constexpr int PY = P == 1 ? 4 : (P == 2 ? 3 : 4);
   static constexpr int cells_per_wave = PX * PY;
   // exchange slot per lane (doubles), even so that slots stay 16-byte
   // aligned for 128-bit LDS accesses; a cell's N slots are followed by a
-  // gap that spreads the cells of a 128-bit read over the banks
-  static constexpr int slot = (NP + 1) & ~1;
+  // gap that spreads the cells of a 128-bit read over the banks. Q3: one
+  // double more than the 16 values (64-bit accesses without conflicts; two
+  // blocks of 4 wavefronts then just fit a compute unit's LDS)
+  static constexpr int slot = P == 3 ? 17 : (NP + 1) & ~1;
   static constexpr int cell_slots = N * slot + (P == 1 ? 2 : 0);
   // slots of every lane's cell, including the partial cell of the lanes
   // past the last whole one (Q2: lane 63 addresses cell 21's planes)
@@ -242,15 +245,14 @@ static __device__ __attribute__((noinline)) void plane_source(
   }
 }
 
-// wavefronts per SIMD the plane kernel is compiled for (VGPR budget)
-#ifndef ADM_PLANE_WAVES_PER_EU
-#define ADM_PLANE_WAVES_PER_EU 2
-#endif
-constexpr int kPlaneWavesPerEU = ADM_PLANE_WAVES_PER_EU;
+// wavefronts per SIMD the plane kernel is compiled for (VGPR budget). Q3
+// holds 16 values per lane where Q2 holds 9: at 2 it spills 200 times per
+// patch (RK4 step of 50x25x17 cells: 236 us against 193 at 1).
+constexpr int plane_waves_per_eu(int p) { return p == 3 ? 1 : 2; }
 
 template <int P, int NS, int PK>
 __global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(ADM_PLANE_WAVES_PER_EU)))
+    __attribute__((amdgpu_waves_per_eu(plane_waves_per_eu(P))))
     plane_kernel(const CellArgs a, const double *__restrict__ src,
                  double *__restrict__ dst) {
   using L = PlaneLanes<P>;
@@ -520,6 +522,22 @@ __global__ void __launch_bounds__(256)
     DS[2][0] = -e02;
     DS[2][1] = -e01;
     DS[2][2] = -e00;
+  } else if constexpr (P == 3) {
+    // S as it is (the values at the points are the oracle's bit for bit); of
+    // the derivative tables one half, made antisymmetric on the host
+#pragma unroll
+    for (int q = 0; q < N; ++q)
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        S[q][k] = in_sgpr(kc.S[q][k]);
+        if (q < N / 2) {
+          Dc[q][k] = in_sgpr(kc.aDc[q][k]);
+          DS[q][k] = in_sgpr(kc.aDcS[q][k]);
+        } else {
+          Dc[q][k] = -Dc[N - 1 - q][N - 1 - k];
+          DS[q][k] = -DS[N - 1 - q][N - 1 - k];
+        }
+      }
   } else {
 #pragma unroll
     for (int q = 0; q < N; ++q)

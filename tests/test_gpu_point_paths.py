@@ -25,6 +25,18 @@ def field(p, kind):
     return 290.0 + 2900.0 * X[:, 0] + 8.0 * s  # below to above the tables
 
 
+def four_materials(m):
+    import copy
+    out = copy.deepcopy(m)
+    out.n_materials = 4
+    out.single_material_layout = False
+    for k in range(1, 4):
+        out.table[k] = m.table[0]
+        out.table[k, :, :, :, 1] *= 1.0 + 0.1 * k
+        out.prop[k] = m.prop[0]
+    return out
+
+
 def problem(degree, cells, variant):
     p = plain_large(n_cells=cells)
     p.fe_degree = degree
@@ -40,6 +52,9 @@ def problem(degree, cells, variant):
         ang = rng.uniform(0.0, 3.0, p.n_cells_total)
         ang[rng.rand(p.n_cells_total) < 0.3] = 0.0
         p.deposition_cos, p.deposition_sin = np.cos(ang), np.sin(ang)
+    if variant == "materials":  # four sets of tables, mixed by cell
+        p.cell_material = rng.randint(0, 4, p.n_cells_total).astype(np.uint8)
+        m = p.material = four_materials(p.material)
     if variant == "anisotropic":
         m = p.material
         for s, f in (("solid", 1.0), ("liquid", 1.0), ("powder", 0.01)):
@@ -50,7 +65,7 @@ def problem(degree, cells, variant):
 
 
 @pytest.mark.parametrize("variant", ["plain", "mixed", "rotated",
-                                     "anisotropic"])
+                                     "anisotropic", "materials"])
 @pytest.mark.parametrize("kind", ["cold", "breaks", "melt"])
 @pytest.mark.parametrize("degree,cells", [
     (1, (1, 1, 1)), (1, (8, 4, 2)), (1, (17, 5, 3)),
