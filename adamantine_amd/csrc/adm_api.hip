@@ -1382,6 +1382,13 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
     } else {
       ac.plane_E = ensure_patch_buffer((size_t)ac.plane_E_stride * M);
     }
+    // One operator: the face term's blocks ride at the end of the patches'
+    // launch (RK4 step of 64x32x12 Q2: 120 us with a launch of its own, 104
+    // so). Batched members keep the launch: a member's face blocks would come
+    // before the next member's patches, whose blocks then start late (64
+    // members: 2.39 ms per step with a launch of its own, 3.01 so).
+    FaceArgs pf = fa;
+    if (M > 1) pf.n_faces = 0;
     if (ac.n_rows > 0) {
       // a persistent grid: 2 wavefronts per SIMD, as many blocks as the
       // chip holds at the occupancy of Q1 and Q2 (shared among the
@@ -1396,11 +1403,11 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
 #define ADM_DISPATCH(P_, NS_)                                              \
   if (p == P_ && n_states == NS_) {                                         \
     if (pk == 0)                                                            \
-      launch_plane<P_, NS_, 0>(ac, src, dst, nb, plds, M, cell_waves, s);   \
+      launch_plane<P_, NS_, 0>(ac, pf, src, nb, plds, M, cell_waves, s);    \
     else if (pk == 1)                                                       \
-      launch_plane<P_, NS_, 1>(ac, src, dst, nb, plds, M, cell_waves, s);   \
+      launch_plane<P_, NS_, 1>(ac, pf, src, nb, plds, M, cell_waves, s);    \
     else                                                                    \
-      launch_plane<P_, NS_, 2>(ac, src, dst, nb, plds, M, cell_waves, s);   \
+      launch_plane<P_, NS_, 2>(ac, pf, src, nb, plds, M, cell_waves, s);    \
   }
       ADM_DISPATCH(1, 1)
       ADM_DISPATCH(1, 2)
@@ -1413,9 +1420,9 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
       ADM_DISPATCH(3, 3)
 #undef ADM_DISPATCH
     }
-    // the face term's slots, then the second pass: every node's sum from
-    // the patch buffer and its face slots into dst
-    launch_faces();
+    // the second pass: every node's sum from the patch buffer and its face
+    // slots into dst
+    if (M > 1 || ac.n_rows == 0) launch_faces();
     // a stage update leaves the nodes above the active cell layers as they
     // are (the gather returns at once there), so its grid stops at them;
     // dst = A src is zero there and is written

@@ -22,18 +22,23 @@ void launch_cell(const CellArgs &a, const double *src, double *dst,
 
 #if ADM_P <= 3
 template <int P, int NS, int PK>
-void launch_plane(const CellArgs &a, const double *src, double *dst,
+void launch_plane(const CellArgs &a, const FaceArgs &fa, const double *src,
                   int64_t n_blocks, size_t lds_bytes, unsigned n_members,
                   int waves, hipStream_t s) {
   const size_t xbytes = sizeof(double) * waves * a.plane_wave_lds;
-  hipLaunchKernelGGL((plane_kernel<P, NS, PK>), dim3((unsigned)n_blocks,
-                     n_members), dim3(64 * waves), lds_bytes + xbytes, s, a,
-                     src, dst);
+  // and the blocks of the face term
+  const int64_t per = (int64_t)waves * FaceLanes<P>::faces_per_wave;
+  const unsigned grid = (unsigned)(n_blocks + (fa.n_faces + per - 1) / per);
+  CellArgs ac = a;
+  ac.plane_blocks = (int32_t)n_blocks;
+  hipLaunchKernelGGL((plane_kernel<P, NS, PK>), dim3(grid, n_members),
+                     dim3(64 * waves), lds_bytes + xbytes, s, ac, src, fa);
 }
 template void launch_plane<ADM_P, ADM_NS, ADM_PK>(const CellArgs &,
-                                                  const double *, double *,
-                                                  int64_t, size_t, unsigned,
-                                                  int, hipStream_t);
+                                                  const FaceArgs &,
+                                                  const double *, int64_t,
+                                                  size_t, unsigned, int,
+                                                  hipStream_t);
 #endif
 
 template <int P, int NS, int PK>

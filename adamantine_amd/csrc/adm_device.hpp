@@ -184,6 +184,7 @@ struct CellArgs {
   // per patch, plane_E_stride per ensemble member) for the gather kernel
   int32_t plane_npx, plane_npy;
   int32_t plane_wave_lds;  // doubles of LDS per wavefront
+  int32_t plane_blocks;    // blocks that take patches (the rest: faces)
   int32_t reach_lo[3], reach_hi[3];  // beam_reach of the launch's beams
   double *plane_E;
   int64_t plane_E_stride;

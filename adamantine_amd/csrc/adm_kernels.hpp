@@ -49,6 +49,7 @@ __device__ __forceinline__ void sweep(const double (&M)[kMaxN][kMaxN],
 // data global (not flat) loads, which LDS waits do not have to wait for.
 #define ADM_GLOBAL __attribute__((address_space(1)))
 #define ADM_CONSTANT __attribute__((address_space(4)))
+#define ADM_LDS __attribute__((address_space(3)))
 template <class T>
 __device__ __forceinline__ ADM_GLOBAL T *as_global(T *p) {
   return (ADM_GLOBAL T *)p;
@@ -124,47 +125,41 @@ struct FaceLanes {
   static constexpr int faces_per_block = 4 * faces_per_wave;
 };
 
+// A block of `waves` wavefronts of the face term, the block-th of the launch;
+// xf: waves * faces_per_wave * (p+1)^2 doubles of LDS. Not inlined: the plane
+// kernel has blocks of its own for it, whose registers it would otherwise
+// take part in.
 template <int P, int NS, int PK>
-__global__ void __launch_bounds__(256)
-    face_kernel(const FaceArgs a, const double *__restrict__ src,
-                double *__restrict__ dst) {
+static __device__ __attribute__((noinline)) void face_block(
+    const ADM_GLOBAL FaceRef *faces, int64_t n_faces,
+    ADM_GLOBAL double *face_powder, ADM_GLOBAL double *face_out,
+    const ADM_GLOBAL KConst *kcp, int nc0, int nc1, int nn0, int nn1,
+    const ADM_GLOBAL double *src, ADM_LDS double *xf, int block, int waves) {
   constexpr int N = P + 1, NF = N * N;
   constexpr int FPW = FaceLanes<P>::faces_per_wave;
-  __shared__ double xf[4][FPW * NF];
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
   const int jf = lane / NF, q = lane % NF;
   const int qa = q % N, qb = q / N;
-  const ADM_CONSTANT MemberArgs *mb =
-      a.members ? as_constant(a.members) + blockIdx.y : nullptr;
-  ADM_GLOBAL double *face_out = as_global(mb ? mb->face_out : a.face_out);
-  const int64_t fi = ((int64_t)blockIdx.x * 4 + wave) * FPW + jf;
+  const int64_t fi = ((int64_t)block * waves + wave) * FPW + jf;
   // whole faces (all lanes of a face) agree
-  if (jf >= FPW || fi >= (mb ? mb->n_faces : a.n_faces)) return;
-  const KConst &kc = *(const KConst *)as_global(mb ? mb->kc : a.kc);
+  if (jf >= FPW || fi >= n_faces) return;
+  const KConst &kc = *(const KConst *)kcp;
   const MatConst &m = kc.mat;
-  const ADM_GLOBAL FaceRef *frp = as_global(mb ? mb->faces : a.faces) + fi;
   FaceRef fr;
-  fr.cell = frp->cell;
-  fr.info = frp->info;
-  ADM_GLOBAL double *face_powder =
-      as_global(mb ? mb->face_powder : a.face_powder);
-  if (mb) {
-    src += (int64_t)blockIdx.y * a.member_stride;
-    dst += (int64_t)blockIdx.y * a.member_stride;
-  }
+  fr.cell = faces[fi].cell;
+  fr.info = faces[fi].info;
   const int64_t c = fr.cell;
   const int f = fr.info & 7, bt = (fr.info >> 3) & 31, mid = (fr.info >> 8) & 3;
   const int d = f / 2, side = f % 2;
-  const int cc[3] = {(int)(c % a.nc[0]), (int)((c / a.nc[0]) % a.nc[1]),
-                     (int)(c / ((int64_t)a.nc[0] * a.nc[1]))};
-  const int64_t ns[3] = {1, (int64_t)a.nn[0],
-                         (int64_t)a.nn[0] * (int64_t)a.nn[1]};
+  const int cc[3] = {(int)(c % nc0), (int)((c / nc0) % nc1),
+                     (int)(c / ((int64_t)nc0 * nc1))};
+  const int64_t ns[3] = {1, (int64_t)nn0, (int64_t)nn0 * (int64_t)nn1};
   const int64_t base = (int64_t)cc[0] * P + ns[1] * cc[1] * P +
                        ns[2] * cc[2] * P + (side ? P : 0) * ns[d];
   const int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
   // this lane's node (face-local index q = a + N b)
   const int64_t node = base + qa * ns[t1] + qb * ns[t2];
-  double *fx = &xf[wave][jf * NF];
+  ADM_LDS double *fx = xf + (wave * FPW + jf) * NF;
   fx[q] = src[node];
   wave_lds_sync();
   // T at point (qa, qb): ft[b] = sum_k S[qa][k] u[k + N b], then along b
@@ -211,6 +206,22 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
   for (int i = 1; i < N; ++i) out = __builtin_fma(kc.S[i][qa], ft[i], out);
   face_out[fi * NF + q] = out;
+}
+
+template <int P, int NS, int PK>
+__global__ void __launch_bounds__(256)
+    face_kernel(const FaceArgs a, const double *__restrict__ src,
+                double *__restrict__ dst) {
+  __shared__ double xf[4 * FaceLanes<P>::faces_per_wave * (P + 1) * (P + 1)];
+  const ADM_CONSTANT MemberArgs *mb =
+      a.members ? as_constant(a.members) + blockIdx.y : nullptr;
+  if (mb) src += (int64_t)blockIdx.y * a.member_stride;
+  face_block<P, NS, PK>(
+      as_global(mb ? mb->faces : a.faces), mb ? mb->n_faces : a.n_faces,
+      as_global(mb ? mb->face_powder : a.face_powder),
+      as_global(mb ? mb->face_out : a.face_out),
+      as_global(mb ? mb->kc : a.kc), a.nc[0], a.nc[1], a.nn[0], a.nn[1],
+      as_global(src), (ADM_LDS double *)xf, blockIdx.x, 4);
 }
 
 // Second pass of the face term: one lane per boundary node adds its faces'

@@ -16,11 +16,12 @@ void launch_cell(const CellArgs &a, const double *src, double *dst,
                  int64_t n_blocks, size_t lds_bytes, unsigned n_members,
                  int waves, hipStream_t s);
 
-// The plane kernel (FE degrees 1 and 2 only): one launch of n_blocks
+// The plane kernel (FE degrees 1 to 3): one launch of n_blocks
 // persistent blocks of `waves` wavefronts looping over PX x PY cell
-// patches, their node sums into the patch buffer (no atomics).
+// patches, their node sums into the patch buffer (no atomics), and the
+// blocks of the face term (face_kernel's work).
 template <int P, int NS, int PK>
-void launch_plane(const CellArgs &a, const double *src, double *dst,
+void launch_plane(const CellArgs &a, const FaceArgs &fa, const double *src,
                   int64_t n_blocks, size_t lds_bytes, unsigned n_members,
                   int waves, hipStream_t s);
 
