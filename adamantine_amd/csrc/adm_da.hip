@@ -112,17 +112,20 @@ static double dist3(const double a[3], const double b[3]) {
 // 2.2 ms before, with strided sums and a division per product; the whole
 // analysis 0.89 ms now), written so that every inner loop runs
 // over contiguous values of independent entries; each function has a body
-// for any x86-64 and the same one for AVX2 (chosen when it runs).
+// for any x86-64 and one for AVX2 with FMA (chosen when it runs).
 #define ADM_BODY static inline __attribute__((always_inline))
 
-// y -= f x
+// y -= f x (FMA: with one rounding, where the processor has the instruction)
+template <bool FMA>
 ADM_BODY void axmy(size_t n, double f, const double *__restrict__ x,
                    double *__restrict__ y) {
-  for (size_t k = 0; k < n; ++k) y[k] -= f * x[k];
+  for (size_t k = 0; k < n; ++k)
+    y[k] = FMA ? __builtin_fma(-f, x[k], y[k]) : y[k] - f * x[k];
 }
 
 // LU with partial pivoting: A X = B with B m x nrhs, both row-major and
 // overwritten. False if a pivot is zero.
+template <bool FMA>
 ADM_BODY bool lu_body(int m, double *A, int nrhs, double *B) {
   const size_t M = m, R = nrhs;
   for (size_t c = 0; c < M; ++c) {
@@ -138,13 +141,13 @@ ADM_BODY bool lu_body(int m, double *A, int nrhs, double *B) {
     for (size_t r = c + 1; r < M; ++r) {
       const double f = A[r * M + c] * inv;
       if (f == 0.0) continue;
-      axmy(M - c - 1, f, A + c * M + c + 1, A + r * M + c + 1);
-      axmy(R, f, B + c * R, B + r * R);
+      axmy<FMA>(M - c - 1, f, A + c * M + c + 1, A + r * M + c + 1);
+      axmy<FMA>(R, f, B + c * R, B + r * R);
     }
   }
   for (size_t r = M; r-- > 0;) {
     for (size_t k = r + 1; k < M; ++k)
-      axmy(R, A[r * M + k], B + k * R, B + r * R);
+      axmy<FMA>(R, A[r * M + k], B + k * R, B + r * R);
     const double d = A[r * M + r];
     for (size_t k = 0; k < R; ++k) B[r * R + k] = B[r * R + k] / d;
   }
@@ -153,34 +156,36 @@ ADM_BODY bool lu_body(int m, double *A, int nrhs, double *B) {
 
 // C (p x q, row-major) = sum over k of X[k][a] Y[k][b] (both row-major with
 // m rows): rank-one updates, k in order
+template <bool FMA>
 ADM_BODY void gram_body(int m, int p, const double *X, int q, const double *Y,
                         double *C) {
   std::fill(C, C + (size_t)p * q, 0.0);
   for (int a = 0; a < p; ++a)
     for (int k = 0; k < m; ++k)
-      axmy(q, -X[(size_t)k * p + a], Y + (size_t)k * q, C + (size_t)a * q);
+      axmy<FMA>(q, -X[(size_t)k * p + a], Y + (size_t)k * q, C + (size_t)a * q);
 }
 
 static bool lu_plain(int m, double *A, int nrhs, double *B) {
-  return lu_body(m, A, nrhs, B);
+  return lu_body<false>(m, A, nrhs, B);
 }
 static void gram_plain(int m, int p, const double *X, int q, const double *Y,
                        double *C) {
-  gram_body(m, p, X, q, Y, C);
+  gram_body<false>(m, p, X, q, Y, C);
 }
 #if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
-__attribute__((target("avx2"))) static bool lu_avx2(int m, double *A,
+__attribute__((target("avx2,fma"))) static bool lu_avx2(int m, double *A,
                                                     int nrhs, double *B) {
-  return lu_body(m, A, nrhs, B);
+  return lu_body<true>(m, A, nrhs, B);
 }
-__attribute__((target("avx2"))) static void gram_avx2(int m, int p,
+__attribute__((target("avx2,fma"))) static void gram_avx2(int m, int p,
                                                       const double *X, int q,
                                                       const double *Y,
                                                       double *C) {
-  gram_body(m, p, X, q, Y, C);
+  gram_body<true>(m, p, X, q, Y, C);
 }
 static bool has_avx2() {
-  static const bool yes = __builtin_cpu_supports("avx2");
+  static const bool yes = 
+      __builtin_cpu_supports("avx2") && __builtin_cpu_supports("fma");
   return yes;
 }
 #else
