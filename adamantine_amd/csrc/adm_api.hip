@@ -2371,7 +2371,7 @@ static int check_launch_config(const adm::Context &c, int32_t mode,
     return adm::set_error(ADM_ERR_INVALID, "unknown launch mode");
   if (mode == ADM_LAUNCH_PLANE && p > 2)
     return adm::set_error(ADM_ERR_UNSUPPORTED,
-                          "the plane kernel exists for FE degrees 1 and 2");
+                          "the plane mode can be set for FE degrees 1 and 2");
   if (mode == ADM_LAUNCH_PLANE && n_dofs >= (int64_t)INT32_MAX)
     return adm::set_error(ADM_ERR_UNSUPPORTED,
                           "the plane kernel takes fewer than 2^31 nodes");

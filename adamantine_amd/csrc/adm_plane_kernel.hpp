@@ -46,13 +46,14 @@
 //    flight before it;
 //  - the two parts of the integration share one exchange.
 // 128x64x32 Q2, per application (plane + gather + face kernels): 100.4 us
-// before, 76.9 us with these; 64 members of 64x32x16, per RK4 step: 3.17 ms
-// before, 2.39 ms; Q1 101x67x33: 38.6 us before, 28.6 us. Q3 (line kernel in
-// 8 colour launches before), RK4 step of 50x25x17: 433 us before, 193 us. What is left of the
+// before, 76.9 us with these (71.4 with the face term in the launch); 64
+// members of 64x32x16, per RK4 step: 3.17 ms before, 2.39 ms; Q1 101x67x33:
+// 38.6 us before, 28.6 us (24.5). Q3 (line kernel in 8 colour launches
+// before), RK4 step of 50x25x17: 433 us before, 162 us. What is left of the
 // large launch is its slowest wavefront (melt under the beam: 133,000 cycles
 // against a mean of 87,000). Handing patches out by a counter instead of a
-// fixed share took 73 us there, but the counter's round trip cost the short
-// Q1 patches 10 % and batched launches 2 %.
+// fixed share took 73 us against 77 there, but the counter's round trip cost
+// the short Q1 patches 10 % and batched launches 2 %.
 // Wavefronts that are solid across several intervals (one material, no
 // powder, below the solidus) take a path of their own: the mixtures reduce
 // to the solid value (the reference adds the other states with a zero ratio,
