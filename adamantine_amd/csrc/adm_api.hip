@@ -1227,6 +1227,22 @@ void Context::set_time(double t) {
   }
 }
 
+// the plane kernel's patch shape and LDS for FE degree p
+struct PlaneShape {
+  int px, py, wave_lds, wave_lds_aniso;
+  int64_t patch_nodes;
+};
+template <int P>
+static PlaneShape plane_shape_of() {
+  using L = PlaneLanes<P>;
+  return {L::PX, L::PY, L::wave_lds, L::wave_lds_aniso, L::patch_nodes};
+}
+static PlaneShape plane_shape(int p) {
+  return p == 1   ? plane_shape_of<1>()
+         : p == 2 ? plane_shape_of<2>()
+                  : plane_shape_of<3>();
+}
+
 CellArgs Context::cell_args() const {
   CellArgs a;
   std::memset(&a, 0, sizeof(a));
@@ -1248,6 +1264,11 @@ CellArgs Context::cell_args() const {
   a.sources_on = sources_on ? 1 : 0;
   a.n_cells = n_cells;
   for (size_t b = 0; b < beams.size(); ++b) a.beams[b] = beam_states[b];
+  if (p <= kPlaneMaxDegree) {
+    const PlaneShape shape = plane_shape(p);
+    a.plane_wave_lds =
+        all_isotropic() ? shape.wave_lds : shape.wave_lds_aniso;
+  }
   return a;
 }
 
@@ -1276,22 +1297,6 @@ void Context::apply(const double *src, double *dst, int add, hipStream_t s,
   CellArgs a = cell_args();
   a.add = add;
   launch(a, face_args(), src, dst, 1, s, nz_active, patch);
-}
-
-// the plane kernel's patch shape and LDS for FE degree p
-struct PlaneShape {
-  int px, py, wave_lds, wave_lds_aniso;
-  int64_t patch_nodes;
-};
-template <int P>
-static PlaneShape plane_shape_of() {
-  using L = PlaneLanes<P>;
-  return {L::PX, L::PY, L::wave_lds, L::wave_lds_aniso, L::patch_nodes};
-}
-static PlaneShape plane_shape(int p) {
-  return p == 1   ? plane_shape_of<1>()
-         : p == 2 ? plane_shape_of<2>()
-                  : plane_shape_of<3>();
 }
 
 // Cell and face kernels of the context's configuration; with n_members > 1
@@ -1368,8 +1373,6 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
       beam_reach(ac.beams, ac.n_beams, kc.origin, kc.inv_h, ac.reach_lo,
                  ac.reach_hi);
     }
-    ac.plane_wave_lds =
-        all_isotropic() ? shape.wave_lds : shape.wave_lds_aniso;
     ac.plane_E_stride = (int64_t)ac.n_rows * slots;
     if (patch) {
       if ((size_t)ac.plane_E_stride * M > kNoAllocScratchDoubles)
@@ -1959,6 +1962,7 @@ void Ensemble::refresh_members() {
   std::vector<MemberArgs> h(n);
   max_faces = 0;
   max_fnodes = 0;
+  plane_wave_lds = 0;
   for (int j = 0; j < n; ++j) {
     const Context &c = *members[j];
     if (c.property_kind() != c0.property_kind())
@@ -1985,6 +1989,7 @@ void Ensemble::refresh_members() {
     m.fn_slot = c.d_fn_slot;
     m.n_fnodes = c.n_fnodes;
     m.fn_rank = c.d_fn_rank;
+    plane_wave_lds = std::max(plane_wave_lds, a.plane_wave_lds);
     max_fnodes = std::max(max_fnodes, m.n_fnodes);
     for (size_t b = 0; b < c.beams.size(); ++b)
       m.beam_gain[b] =
@@ -2050,6 +2055,7 @@ CellArgs Ensemble::cell_args(int add) const {
   a.add = add;
   a.members = d_members;
   a.member_stride = n_dofs;
+  a.plane_wave_lds = plane_wave_lds;
   for (int b = 0; b < ADM_MAX_BEAMS; ++b) {
     a.beam_pmod[b] = pmod[b];
     a.beam_den[b] = den[b];

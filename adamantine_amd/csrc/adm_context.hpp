@@ -338,6 +338,10 @@ struct Ensemble {
   int64_t n_dofs = 0;
   int64_t max_faces = 0;
   int64_t max_fnodes = 0;
+  // CellArgs::plane_wave_lds that holds every member: a member's scaled
+  // tables can be isotropic where another's, a last bit apart between the
+  // axes, are not
+  int32_t plane_wave_lds = 0;
   std::vector<std::unique_ptr<Context>> members;
   MemberArgs *d_members = nullptr;
   double pmod[ADM_MAX_BEAMS] = {0, 0, 0, 0};

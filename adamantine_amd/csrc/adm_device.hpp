@@ -183,7 +183,9 @@ struct CellArgs {
   // patch buffer the kernel writes its nodes' sums to (plane_slots doubles
   // per patch, plane_E_stride per ensemble member) for the gather kernel
   int32_t plane_npx, plane_npy;
-  int32_t plane_wave_lds;  // doubles of LDS per wavefront
+  // doubles of LDS per wavefront: more where a material of the operator, or
+  // of any member of the ensemble, is anisotropic
+  int32_t plane_wave_lds;
   int32_t plane_blocks;    // blocks that take patches (the rest: faces)
   int32_t reach_lo[3], reach_hi[3];  // beam_reach of the launch's beams
   double *plane_E;
