@@ -1950,7 +1950,7 @@ Ensemble::Ensemble(const adm_problem_desc &base, int n,
   n_dofs = members[0]->n_dofs;
   auto work = std::make_shared<ActWork>();
   for (auto &m : members) m->act = work;
-  members[0]->reserve_patch_buffer(n);
+  members[0]->reserve_patch_buffer(members[0]->launch_mode(), n);
   refresh_members();
 }
 
@@ -2274,7 +2274,7 @@ int adm_create(const adm_problem_desc *desc, void **out) {
   ADM_API_BEGIN
   if (!desc || !out) return adm::set_error(ADM_ERR_INVALID, "null argument");
   auto ctx = std::make_unique<Context>(*desc);
-  ctx->reserve_patch_buffer(1);
+  ctx->reserve_patch_buffer(ctx->launch_mode(), 1);
   *out = ctx.release();
   ADM_API_END
 }
@@ -2366,24 +2366,23 @@ int adm_vmult(void *ptr, const double *src, double *dst, int add,
   ADM_API_END
 }
 
-// checks a launch configuration for a context of FE degree p
+// checks a launch configuration for a context
 static int check_launch_config(const adm::Context &c, int32_t mode,
                                int32_t waves) {
-  const int p = c.p;
   const int64_t n_dofs = c.n_dofs;
   if (waves < 2 || waves > 4)
     return adm::set_error(ADM_ERR_INVALID, "waves_per_block must be 2..4");
   if (mode < ADM_LAUNCH_LINE_ATOMIC || mode > ADM_LAUNCH_PLANE)
     return adm::set_error(ADM_ERR_INVALID, "unknown launch mode");
-  if (mode == ADM_LAUNCH_PLANE && p > 2)
+  if (mode == ADM_LAUNCH_PLANE && c.p > adm::kPlaneMaxDegree)
     return adm::set_error(ADM_ERR_UNSUPPORTED,
-                          "the plane mode can be set for FE degrees 1 and 2");
+                          "the plane kernel exists for FE degrees 1 to 3");
   if (mode == ADM_LAUNCH_PLANE && n_dofs >= (int64_t)INT32_MAX)
     return adm::set_error(ADM_ERR_UNSUPPORTED,
                           "the plane kernel takes fewer than 2^31 nodes");
   if (mode == ADM_LAUNCH_PLANE && !c.plane_tables_ok)
     return adm::set_error(ADM_ERR_UNSUPPORTED,
-                          "the plane kernel needs the symmetric Q2 tables");
+                          "the plane kernel needs symmetric 1-D tables");
   if (mode == ADM_LAUNCH_PLANE && c.dim == 2)
     return adm::set_error(ADM_ERR_UNSUPPORTED,
                           "the plane kernel is three-dimensional");
@@ -2425,6 +2424,7 @@ int adm_set_launch_config(void *ptr, int32_t mode, int32_t waves_per_block) {
   if (int e = check_launch_config(ctx, mode, waves_per_block))
     return e;
   ADM_HIP(hipDeviceSynchronize());
+  ctx.reserve_patch_buffer(mode, 1);
   ctx.set_launch_mode(mode);
   ctx.cell_waves = waves_per_block;
   ADM_API_END
@@ -2481,6 +2481,7 @@ static void tune_launch(adm::Context &cfg,
         if (ms_out) ms_out[k] = -1.0;
         continue;
       }
+      cfg.reserve_patch_buffer(mode, (unsigned)holders.size());
       cfg.set_launch_mode(mode);
       cfg.cell_waves = w;
       apply();  // warm-up
@@ -2774,6 +2775,7 @@ int adm_ensemble_set_launch_config(void *ptr, int32_t mode,
   if (int e = check_launch_config(*ens.members[0], mode, waves_per_block))
     return e;
   ADM_HIP(hipDeviceSynchronize());
+  ens.members[0]->reserve_patch_buffer(mode, (unsigned)ens.n_members);
   ens.members[0]->set_launch_mode(mode);
   ens.members[0]->cell_waves = waves_per_block;
   ADM_API_END

@@ -184,10 +184,11 @@ struct Context {
   size_t patch_buffer_size(int nz_rows, unsigned n_members) const;
   // the cell term goes through the plane kernel (which writes every node)
   bool plane_path() const { return use_plane && p <= kPlaneMaxDegree; }
-  // Q3: the patch buffer of every cell layer, when the operator is created
-  // (its vmult allocates nothing later, also not while a stream is captured)
-  void reserve_patch_buffer(unsigned n_members) const {
-    if (p == 3 && plane_path())
+  // Q3: the patch buffer of every cell layer, when the operator is created or
+  // the plane mode is set (its vmult allocates nothing later, also not while
+  // a stream is captured)
+  void reserve_patch_buffer(int mode, unsigned n_members) const {
+    if (p == 3 && mode == ADM_LAUNCH_PLANE)
       ensure_patch_buffer(patch_buffer_size(-1, n_members));
   }
   void compute_inverse_mass(double *out, hipStream_t s);
@@ -256,7 +257,8 @@ struct Context {
   // plane kernel (FE degrees 1 to 3; the default there unless
   // ADM_CELL_KERNEL=line is in the environment at creation)
   bool use_plane = false;
-  // the 1-D tables have the symmetries the plane kernel's Q2 form uses
+  // the 1-D tables have the symmetries the plane kernel uses: weights at
+  // every degree, S and Dc at degree 2
   bool plane_tables_ok = true;
   // ADM_LAUNCH_* mode of the fields above
   int launch_mode() const {

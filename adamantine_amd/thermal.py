@@ -244,7 +244,7 @@ class ThermalOperatorDevice:
     # quadrature-point state --------------------------------------------------
     def set_launch_config(self, mode: int, waves_per_block: int):
         """mode: LAUNCH_LINE_ATOMIC (0), LAUNCH_LINE_COLORED (1) or
-        LAUNCH_PLANE (2, FE degrees 1 and 2); 2..4 wavefronts per block."""
+        LAUNCH_PLANE (2, 3-D FE degrees 1 to 3); 2..4 wavefronts per block."""
         check(load_library().adm_set_launch_config(
             self._h, int(mode), int(waves_per_block)))
 

@@ -306,22 +306,24 @@ int adm_vmult_noalloc(void *ctx, const double *src, double *dst, int add,
 #define ADM_LAUNCH_LINE_ATOMIC 0  /* line kernel, one launch, FP64 atomics */
 #define ADM_LAUNCH_LINE_COLORED 1 /* line kernel, 8 parity-colour launches
                                      with plain read-add-write */
-#define ADM_LAUNCH_PLANE 2        /* plane kernel (FE degree 1 or 2 only):
-                                     one launch, shared nodes summed in the
-                                     wavefront, then atomics */
+#define ADM_LAUNCH_PLANE 2        /* plane kernel (FE degrees 1 to 3): one
+                                     launch, shared nodes summed in the
+                                     wavefront, then by a gather pass over a
+                                     patch buffer (no atomics) */
 #define ADM_N_LAUNCH_CONFIGS 9    /* 3 modes x 2..4 wavefronts per block */
 
 /* Launch configuration of the cell kernel: one of the ADM_LAUNCH_* modes and
- * 2..4 wavefronts per block (default: the plane kernel for FE degrees 1 and
- * 2, the colour launches of the line kernel otherwise, 4 wavefronts). The
- * plane mode is refused for FE degrees above 2. */
+ * 2..4 wavefronts per block (default: the plane kernel for FE degrees 1 to 3
+ * in three dimensions, the colour launches of the line kernel otherwise, 4
+ * wavefronts). The plane mode is refused for FE degrees above 3 and in two
+ * dimensions. Any mode that adm_autotune returns can be set. */
 int adm_set_launch_config(void *ctx, int32_t mode, int32_t waves_per_block);
 
 /* Autotuner (no reference counterpart): times `reps` vmults of src into dst
  * (device vectors) under each launch configuration (modes 1, 0, 2, each
  * with 2, 3, 4 wavefronts per block; ms_out, host, may be NULL, receives
  * the ADM_N_LAUNCH_CONFIGS per-vmult times in that order, -1 for the plane
- * mode where the FE degree has none), keeps the fastest and returns it.
+ * mode where it is refused), keeps the fastest and returns it.
  * The phase state is restored afterwards, so later results do not depend
  * on the tuning. */
 int adm_autotune(void *ctx, const double *src, double *dst, int32_t reps,

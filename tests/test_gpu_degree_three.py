@@ -1,0 +1,106 @@
+"""FE degree 3 on the routes around its default, the plane kernel: every launch
+mode, set by hand and as a tuner returns it, for one operator and for an
+ensemble, against the oracle. Bars as in test_gpu_parity."""
+import numpy as np
+import pytest
+
+from adamantine_amd.thermal import (LAUNCH_LINE_ATOMIC, LAUNCH_LINE_COLORED,
+                                    LAUNCH_PLANE)
+from adamantine_amd.workloads import (ensemble_workload, plain_large,
+                                      random_temperature)
+from oracle.oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+VMULT_TOL = 1e-12
+MODES = (LAUNCH_LINE_COLORED, LAUNCH_LINE_ATOMIC, LAUNCH_PLANE)
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300)
+
+
+def problem(n_cells=(9, 5, 6)):
+    p = plain_large(n_cells=n_cells)
+    p.fe_degree = 3
+    return p
+
+
+def ensemble(n_members=3):
+    base, members = ensemble_workload(n_members=n_members, n_cells=(9, 5, 8))
+    base.fe_degree = 3
+    return base, members
+
+
+def apply(op, T, t):
+    import torch
+    op.set_time(t)
+    dst = op.initialize_dof_vector(7.0)  # stale contents must not matter
+    op.vmult(dst, torch.tensor(T, device="cuda"))
+    return dst.cpu().numpy()
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("waves", [2, 3, 4])
+def test_launch_modes(mode, waves):
+    """Every mode can be set, and the default taken back after it."""
+    from adamantine_amd.thermal import ThermalOperatorDevice
+    p = problem()
+    T = random_temperature(p, seed=8, low=1200.0, high=2000.0)
+    op, o = ThermalOperatorDevice(p), Oracle(p)
+    o.set_time(1e-4)
+    want = o.vmult(T)
+    first = apply(ThermalOperatorDevice(p), T, 1e-4)
+    op.set_launch_config(mode, waves)
+    assert rel(apply(op, T, 1e-4), want) < VMULT_TOL
+    for a, b in zip(op.qp_state(), o.qp_state()):
+        np.testing.assert_array_equal(a, b)
+    fresh = ThermalOperatorDevice(p)
+    fresh.set_launch_config(mode, waves)
+    fresh.set_launch_config(LAUNCH_PLANE, 4)
+    np.testing.assert_array_equal(apply(fresh, T, 1e-4), first)
+
+
+def test_tuned_mode_sets():
+    """What the tuner returns, set on another operator (as a program that
+    tunes one of several does)."""
+    import torch
+    from adamantine_amd.thermal import ThermalOperatorDevice
+    p = problem()
+    T = random_temperature(p, seed=8, low=1200.0, high=2000.0)
+    a, b, o = ThermalOperatorDevice(p), ThermalOperatorDevice(p), Oracle(p)
+    a.set_time(1e-4)
+    res = a.autotune(torch.tensor(T, device="cuda"), reps=2)
+    assert all(v > 0 for v in res["ms"].values())
+    b.set_launch_config(res["mode"], res["waves_per_block"])
+    o.set_time(1e-4)
+    want = o.vmult(T)
+    for op in (a, b):
+        assert rel(apply(op, T, 1e-4), want) < VMULT_TOL
+
+
+def test_ensemble_modes():
+    import torch
+    from adamantine_amd.ensemble import EnsembleDevice, member_problem
+    base, members = ensemble()
+    T = np.stack([np.random.RandomState(40 + j).uniform(300, 2000,
+                                                        base.n_dofs)
+                  for j in range(len(members))])
+    want, state = [], []
+    for m, u in zip(members, T):
+        o = Oracle(member_problem(base, m))
+        o.set_time(2e-4)
+        want.append(o.vmult(u))
+        state.append(o.qp_state())
+    tuned = EnsembleDevice(base, members)
+    tuned.set_time(2e-4)
+    res = tuned.autotune(torch.tensor(T, device="cuda"), reps=2)
+    configs = [(m, w) for m in MODES for w in (2, 3, 4)]
+    for mode, waves in configs + [(res["mode"], res["waves_per_block"])]:
+        ens = EnsembleDevice(base, members)
+        ens.set_launch_config(mode, waves)
+        got = apply(ens, T, 2e-4)
+        for j in range(len(members)):
+            assert rel(got[j], want[j]) < VMULT_TOL, (mode, waves, j)
+            for a, b in zip(ens.qp_state(j), state[j]):
+                np.testing.assert_array_equal(a, b)
