@@ -2395,25 +2395,18 @@ int adm_vmult_noalloc(void *ptr, const double *src, double *dst, int add,
   ADM_CTX(ptr)
   if (!src || !dst) return adm::set_error(ADM_ERR_INVALID, "null vector");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // as adm_vmult, with the scratch array as the patch buffer; Q3, whose patch
-  // buffer is larger than the array for meshes that this call takes, through
-  // the line kernel
-  struct Line {
-    adm::Context &c;
-    const bool plane;
-    explicit Line(adm::Context &c_) : c(c_), plane(c_.use_plane) {
-      if (c.p == 3) c.use_plane = false;
-    }
-    ~Line() { c.use_plane = plane; }
-  } line(ctx);
+  // as adm_vmult, with the scratch array as the patch buffer; Q3 takes its own
+  // one, which the plane mode has reserved for every cell layer (larger than
+  // the scratch array for meshes that this call takes)
+  double *patch = ctx.p == 3 ? nullptr : ctx.d_scratch;
   if (ctx.n_ext >= 0) {
     ctx.to_nodes(src, ctx.d_map_src, s);
     if (!ctx.plane_path()) ctx.fill(ctx.d_map_dst, 0.0, ctx.n_dofs, s);
-    ctx.apply(ctx.d_map_src, ctx.d_map_dst, 0, s, ctx.d_scratch);
+    ctx.apply(ctx.d_map_src, ctx.d_map_dst, 0, s, patch);
     ctx.to_dofs(ctx.d_map_dst, dst, add, s);
   } else {
     if (!add && !ctx.plane_path()) ctx.fill(dst, 0.0, ctx.n_dofs, s);
-    ctx.apply(src, dst, add, s, ctx.d_scratch);
+    ctx.apply(src, dst, add, s, patch);
   }
   ADM_API_END
 }

@@ -288,16 +288,19 @@ int adm_vmult(void *ctx, const double *src, double *dst, int add,
 /* adm_vmult that allocates nothing. No counterpart in the reference: it is
  * for callers that cannot allocate device memory during the call (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc). adm_vmult may grow the plane kernel's patch buffer with
- * hipMalloc on its first call or after an activation; this entry point
- * uses instead a static device array of the library, 40 MiB per device
- * (5 * 2^20 doubles), held until the process ends, and refuses
+ * hipMalloc). For FE degrees 1 and 2 adm_vmult may grow the plane kernel's
+ * patch buffer with hipMalloc on its first call or after an activation; this
+ * entry point uses instead a static device array of the library, 40 MiB per
+ * device (5 * 2^20 doubles), held until the process ends, and refuses
  * (ADM_ERR_UNSUPPORTED) a mesh whose patch buffer needs more (the
  * 128x64x32 Q2 workload needs 4.2 million doubles). Every call on one
  * device shares that array: calls that overlap on one device (several
  * streams, several host threads) race; calls in one stream, one after the
  * other, are safe (the array needs no clearing: every slot a call reads
- * it writes first). Same arguments and results as adm_vmult. */
+ * it writes first). For degree 3 the operator holds a patch buffer for every
+ * cell layer (about 1.6 doubles per node and member, active or not) from its
+ * creation, or from setting the plane mode, on; both calls use it and neither
+ * allocates. Same arguments and results as adm_vmult. */
 int adm_vmult_noalloc(void *ctx, const double *src, double *dst, int add,
                       void *stream);
 

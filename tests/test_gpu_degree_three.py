@@ -104,3 +104,80 @@ def test_ensemble_modes():
             assert rel(got[j], want[j]) < VMULT_TOL, (mode, waves, j)
             for a, b in zip(ens.qp_state(j), state[j]):
                 np.testing.assert_array_equal(a, b)
+
+
+def noalloc(op, src, dst):
+    from adamantine_amd import thermal as TH
+    TH.check(TH.load_library().adm_vmult_noalloc(
+        op.handle, TH._dev_ptr(src, op.m()), TH._dev_ptr(dst, op.m()), 0,
+        TH._stream_ptr()))
+
+
+@pytest.mark.parametrize("mode", ["default", "tuned", LAUNCH_LINE_COLORED])
+def test_noalloc_is_vmult(mode):
+    """adm_vmult_noalloc gives adm_vmult's bits, whatever mode is set (but
+    the atomic one, whose sums vary), and allocates nothing; the second mesh
+    needs more than the library's scratch array."""
+    import torch
+    from adamantine_amd.thermal import ThermalOperatorDevice
+    # 24 x 12 patches x 32 layers x 676 nodes = 6.2 million doubles
+    for n_cells in ((9, 5, 6), (96, 48, 32)):
+        print("no-alloc vmult, degree 3:", mode, n_cells, flush=True)
+        p = problem(n_cells)
+        T = torch.tensor(random_temperature(p, seed=5, low=300.0,
+                                            high=2000.0), device="cuda")
+        a, b = ThermalOperatorDevice(p), ThermalOperatorDevice(p)
+        if mode == "tuned":
+            res = a.autotune(T, reps=1)
+            if res["mode"] == LAUNCH_LINE_ATOMIC:
+                a.set_launch_config(LAUNCH_PLANE, 4)
+                res["mode"] = LAUNCH_PLANE
+            b.set_launch_config(res["mode"], res["waves_per_block"])
+        elif mode != "default":
+            a.set_launch_config(mode, 4)
+            b.set_launch_config(mode, 4)
+        for t in (0.0, 2e-4):
+            a.set_time(t)
+            b.set_time(t)
+            want = a.initialize_dof_vector(7.0)
+            got = b.initialize_dof_vector(7.0)
+            a.vmult(want, T)
+            torch.cuda.synchronize()
+            free = torch.cuda.mem_get_info()[0]
+            noalloc(b, T, got)
+            torch.cuda.synchronize()
+            assert torch.cuda.mem_get_info()[0] == free
+            assert torch.equal(got, want)
+        for x, y in zip(a.qp_state(), b.qp_state()):
+            np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("call", ["vmult", "noalloc"])
+def test_captured(call):
+    """Both calls under stream capture on an operator that has not run yet:
+    nothing is allocated. Replays with eager work between them."""
+    import torch
+    from adamantine_amd.thermal import ThermalOperatorDevice
+    print("captured", call, "degree 3", flush=True)
+    p = problem()
+    T = torch.tensor(random_temperature(p, seed=5, low=300.0, high=2000.0),
+                     device="cuda")
+    op, twin = ThermalOperatorDevice(p), ThermalOperatorDevice(p)
+    op.set_time(1e-4)
+    twin.set_time(1e-4)
+    src = torch.empty_like(T)
+    dst = op.initialize_dof_vector(7.0)
+    want = twin.initialize_dof_vector(0.0)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        op.vmult(dst, src) if call == "vmult" else noalloc(op, src, dst)
+    for rep in range(4):
+        src.copy_(T + 30.0 * rep)
+        graph.replay()
+        torch.cuda.synchronize()
+        twin.vmult(want, src)
+        torch.cuda.synchronize()
+        assert torch.equal(dst, want), rep
+        dst.fill_(float(rep))
+    for x, y in zip(op.qp_state(), twin.qp_state()):
+        np.testing.assert_array_equal(x, y)
