@@ -52,3 +52,18 @@ def test_localized_update_not_finite():
     assert far.any() and not far.all()
     np.testing.assert_allclose(got[:, far], X[:, far], rtol=1e-14)
     assert not np.isfinite(got[:, obs[0]]).any()
+
+
+def test_localized_update_not_finite_reaches_all():
+    """An observation that is not finite makes the gains of all of them so,
+    also of those out of its reach."""
+    base, ens, X, obs, y, R, noise = setup(5, 3, 3)
+    xyz = base.node_coordinates()
+    obs = np.array([0, ens.n_dofs // 2, ens.n_dofs - 1])
+    assert np.linalg.norm(xyz[obs[0]] - xyz[obs[2]]) > 0.4e-3
+    y[0] = np.inf
+    got = update(ens, base, "gaspari_cohn", 0.4e-3, X, obs, y, R, noise)
+    far = (np.linalg.norm(xyz[:, None] - xyz[obs], axis=2) > 0.4e-3).all(1)
+    assert far.any()
+    np.testing.assert_allclose(got[:, far], X[:, far], rtol=1e-14)
+    assert not np.isfinite(got[:, obs]).any()
