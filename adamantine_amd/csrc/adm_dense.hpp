@@ -16,12 +16,14 @@ namespace adm {
 // for any x86-64 and one for AVX2 with FMA (chosen when it runs).
 #define ADM_BODY static inline __attribute__((always_inline))
 
-// y -= f x (FMA: with one rounding, where the processor has the instruction)
-template <bool FMA>
+// y -= f x, each with one rounding in both bodies: without the instruction
+// the C library's fma gives the same bits, so that an analysis does not depend
+// on the processor (LU of 200 rows, 32 right-hand sides: 0.87 ms with AVX2 and
+// FMA, 11.6 ms in the plain body; the server processors beside this GPU have
+// both)
 ADM_BODY void axmy(size_t n, double f, const double *__restrict__ x,
                    double *__restrict__ y) {
-  for (size_t k = 0; k < n; ++k)
-    y[k] = FMA ? __builtin_fma(-f, x[k], y[k]) : y[k] - f * x[k];
+  for (size_t k = 0; k < n; ++k) y[k] = __builtin_fma(-f, x[k], y[k]);
 }
 
 // (these two are not inlined: rare, beside the loops over rows below)
@@ -33,12 +35,11 @@ static __attribute__((noinline)) int all_finite(size_t n, const double *x) {
 // y -= f x with f = 0: not a number where x is not finite
 static __attribute__((noinline)) void subtract_zero_times(
     size_t n, double f, const double *x, double *y) {
-  for (size_t k = 0; k < n; ++k) y[k] -= f * x[k];
+  for (size_t k = 0; k < n; ++k) y[k] = __builtin_fma(-f, x[k], y[k]);
 }
 
 // LU with partial pivoting: A X = B with B m x nrhs, both row-major and
 // overwritten. False if a pivot is zero.
-template <bool FMA>
 ADM_BODY bool lu_body(int m, double *A, int nrhs, double *B) {
   const size_t M = m, R = nrhs;
   for (size_t c = 0; c < M; ++c) {
@@ -61,13 +62,13 @@ ADM_BODY bool lu_body(int m, double *A, int nrhs, double *B) {
         if (!finite) subtract_zero_times(R, f, B + c * R, B + r * R);
         continue;
       }
-      axmy<FMA>(M - c - 1, f, A + c * M + c + 1, A + r * M + c + 1);
-      axmy<FMA>(R, f, B + c * R, B + r * R);
+      axmy(M - c - 1, f, A + c * M + c + 1, A + r * M + c + 1);
+      axmy(R, f, B + c * R, B + r * R);
     }
   }
   for (size_t r = M; r-- > 0;) {
     for (size_t k = r + 1; k < M; ++k)
-      axmy<FMA>(R, A[r * M + k], B + k * R, B + r * R);
+      axmy(R, A[r * M + k], B + k * R, B + r * R);
     const double d = A[r * M + r];
     for (size_t k = 0; k < R; ++k) B[r * R + k] = B[r * R + k] / d;
   }
@@ -76,30 +77,29 @@ ADM_BODY bool lu_body(int m, double *A, int nrhs, double *B) {
 
 // C (p x q, row-major) = sum over k of X[k][a] Y[k][b] (both row-major with
 // m rows): rank-one updates, k in order
-template <bool FMA>
 ADM_BODY void gram_body(int m, int p, const double *X, int q, const double *Y,
                         double *C) {
   std::fill(C, C + (size_t)p * q, 0.0);
   for (int a = 0; a < p; ++a)
     for (int k = 0; k < m; ++k)
-      axmy<FMA>(q, -X[(size_t)k * p + a], Y + (size_t)k * q, C + (size_t)a * q);
+      axmy(q, -X[(size_t)k * p + a], Y + (size_t)k * q, C + (size_t)a * q);
 }
 
 static bool lu_plain(int m, double *A, int nrhs, double *B) {
-  return lu_body<false>(m, A, nrhs, B);
+  return lu_body(m, A, nrhs, B);
 }
 static void gram_plain(int m, int p, const double *X, int q, const double *Y,
                        double *C) {
-  gram_body<false>(m, p, X, q, Y, C);
+  gram_body(m, p, X, q, Y, C);
 }
 #if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
 __attribute__((target("avx2,fma"))) static bool lu_avx2(int m, double *A,
                                                         int nrhs, double *B) {
-  return lu_body<true>(m, A, nrhs, B);
+  return lu_body(m, A, nrhs, B);
 }
 __attribute__((target("avx2,fma"))) static void gram_avx2(
     int m, int p, const double *X, int q, const double *Y, double *C) {
-  gram_body<true>(m, p, X, q, Y, C);
+  gram_body(m, p, X, q, Y, C);
 }
 static bool has_avx2() {
   static const bool yes =

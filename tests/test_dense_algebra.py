@@ -113,3 +113,23 @@ def test_gram(lib, body, m, p, q):
     lib.gram(body, m, p, ptr(X), q, ptr(Y), ptr(got))
     assert (np.abs(got - X.T @ Y)
             <= 2.0 * m * EPS * (np.abs(X.T) @ np.abs(Y))).all()
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_bodies_agree(lib, seed):
+    """Bit for bit, so that an analysis does not depend on the processor."""
+    if not lib.has_body(1):
+        pytest.skip("the processor has no AVX2")
+    rng = np.random.RandomState(seed)
+    m = 37
+    A = rng.uniform(-1.0, 1.0, (m, m))
+    A[rng.uniform(size=(m, m)) < 0.3] = 0.0  # zero multipliers too
+    A += np.diag(rng.uniform(0.0, 2.0, m))
+    B = rng.uniform(-1.0, 1.0, (m, 19))
+    out = [solve(lib, body, A, B) for body in (0, 1)]
+    assert out[0][0] and out[1][0]
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+    C = [np.empty((m, 19)) for _ in range(2)]
+    for body in (0, 1):
+        lib.gram(body, m, m, ptr(A), 19, ptr(B), ptr(C[body]))
+    np.testing.assert_array_equal(C[0], C[1])
