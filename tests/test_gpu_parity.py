@@ -272,7 +272,8 @@ def test_invalid_arguments():
 
 
 def test_degree_three():
-    """FE degree 3 (16 lanes per cell, 4 cells per wavefront): lumped mass
+    """FE degree 3 on its default route, the plane kernel (4 lanes per cell, 16
+    cells per wavefront; the others: test_gpu_degree_three): lumped mass
     bit-exact, vmult and phase state against the oracle on a SLP table
     problem with powder, rotation and radiative/convective faces, and an RK4
     step."""
