@@ -234,7 +234,7 @@ __device__ __forceinline__ double beam_value_dR(const adm_beam_state &s,
 // latency (two fields' exchanges and the points' table reads); with the 1-D
 // tables and material constants in LDS, the prologue's loads together and the
 // source only where a beam reaches, a gradient of 8 members of 48x24x16 went
-// from 9.34 to 8.84 ms, one of 64x32x12 from 8.74 to 8.50 ms.
+// from 9.34 to 8.84 ms, one of 64x32x12 from 8.74 to 8.53 ms.
 template <int P, int NS, int PK>
 __global__ void __launch_bounds__(256)
     adjoint_cell_kernel(const AdjArgs aa) {

@@ -1387,9 +1387,13 @@ void Context::launch(const CellArgs &a, const FaceArgs &fa, const double *src,
     }
     // One operator: the face term's blocks ride at the end of the patches'
     // launch (RK4 step of 64x32x12 Q2: 120 us with a launch of its own, 104
-    // so). Batched members keep the launch: a member's face blocks would come
-    // before the next member's patches, whose blocks then start late (64
-    // members: 2.39 ms per step with a launch of its own, 3.01 so).
+    // so). Batched members keep the launch: the grid's y index is the member,
+    // so a member's face blocks come before the next member's patches, whose
+    // blocks then start late. Per RK4 step of 64x32x16 Q2, with a launch of
+    // its own and riding: 2 members 166 and 138 us, 4: 230 and 211, 8: 343 and
+    // 363, 16: 602 and 665, 64: 2.15 and 2.86 ms (16x8x8 Q2: riding is 1.18
+    // times faster for 2 to 8 members, 0.92 for 64). Batches of a few members
+    // would gain, but where the sides cross depends on the mesh.
     FaceArgs pf = fa;
     if (M > 1) pf.n_faces = 0;
     if (ac.n_rows > 0) {

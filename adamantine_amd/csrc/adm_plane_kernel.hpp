@@ -8,8 +8,9 @@
 // buffer: one exchange for the evaluation and one for the integration
 // (against six in the line-per-lane kernel). A wavefront takes a patch of
 // PX x PY cells of one cell layer (7 x 3 for Q2: 63 lanes; 8 x 4 for Q1 and
-// 4 x 4 for Q3: 64 lanes), so the nodes its cells share along x and y are summed inside
-// the wavefront (cross-lane shuffles). Each patch then stores its node sums
+// 4 x 4 for Q3: 64 lanes), so the nodes its cells share along x and y are
+// summed inside the wavefront (cross-lane shuffles). Each patch then stores
+// its node sums
 // in its own block of a patch buffer, and a second kernel (one lane per
 // node) adds the blocks of the patches that share the node, in a fixed
 // order, into dst. No atomics: FP64 atomic adds to device memory are
@@ -42,8 +43,10 @@
 //  - the other wavefronts work in two steps with the points' properties in
 //    LDS between them (see there), the heat source sits behind a call and
 //    scalar constants that follow from symmetry are not held twice, so that
-//    nothing spills: one spilled register's reload waits for the loads in
-//    flight before it;
+//    no vector register spills to memory: its reload would wait for the loads
+//    in flight before it. Scalar registers do spill, to lanes of vector
+//    registers (95 for Q1, 102 for Q2, 183 for Q3 with three states and merged
+//    tables);
 //  - the two parts of the integration share one exchange.
 // 128x64x32 Q2, per application (plane + gather + face kernels): 100.4 us
 // before, 76.9 us with these (71.4 with the face term in the launch); 64
