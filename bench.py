@@ -32,7 +32,7 @@ LAUNCH_MODE_NAMES = {0: "line_atomic", 1: "line_colored", 2: "plane"}
 MEASURED_TRAFFIC_BYTES = {
     "line_colored": 355.6e6,
     "line_atomic": 176.0e6,
-    "plane": 127.1e6,
+    "plane": 129.8e6,
 }
 TRAFFIC_PROFILE = {
     "line_colored": "profiles/hbm_traffic_plain_large.md",
