@@ -417,11 +417,42 @@ static void launch_transform(int NT, double *X, const double *Tm, int N,
   ADM_HIP_DA(hipGetLastError());
 }
 
-static void launch_localized(bool finite, double *T, int N, int64_t n,
+// Which localised kernel costs less. Estimates per node, in units of one
+// distance test of the lane-per-node kernel:
+//   lane per node: 4.5 + m (1 + f (1 + 2/3 N)), f the share of observations
+//     that a node's wavefront reaches (the cut-off's box over the mesh's);
+//     with fewer than 500,000 nodes the chip is not full and the launch
+//     lasts as long as with as many;
+//   matrix tiles: 10 + (24 + 56 g) per 16 observations, however few of them
+//     there are, g the chance that a tile is within the cut-off.
+// Whole analyses, lane and matrix kernel: 2 members, 1 observation,
+// 2,154,945 nodes 75 and 201 us; 16 members, 128 observations, cut-off
+// 0.2 mm of a 4 x 2 x 1 mm box, 2,154,945 nodes 488 and 637 us; 17 members,
+// 1 observation, 276,705 nodes 72 and 83 us; 8 members, 32 observations,
+// cut-off 3 mm, 276,705 nodes 113 and 88 us, 20,825 nodes 105 and 61 us. Over
+// 2,020 such pairs (2 to 32 members, 1 to 128 observations, 4,913 to
+// 2,154,945 nodes) the choice is the faster one or loses 0.3 % on average,
+// 13 % at most; above 32 members the lane kernel was never the faster one
+// (1.3 to 8.6 times slower, 4,913 and 276,705 nodes).
+static bool localized_mfma_pays(int N, int64_t n, int m, double cutoff,
+                                const NodeGeometry &geo) {
+  if (N > 32) return true;
+  double f = 1.0;
+  for (int d = 0; d < 3; ++d)
+    if (geo.nn[d] > 1)
+      f *= std::min(1.0, 2.0 * cutoff / (geo.h[d] * geo.nc[d]));
+  const double g = 1.0 - std::pow(1.0 - f, 16);
+  const double lane = std::max((double)n, 5e5) *
+                      (4.5 + m * (1.0 + f * (1.0 + 2.0 / 3.0 * N)));
+  const double tiles = (double)n * (10.0 + (m + 15) / 16 * (24.0 + 56.0 * g));
+  return tiles < lane;
+}
+
+static void launch_localized(bool tiles, double *T, int N, int64_t n,
                              const double *S, const double *E,
                              const double *oc, int m, int fn, double cutoff,
                              const NodeGeometry &geo, hipStream_t s) {
-  if (finite) {
+  if (tiles) {
     const unsigned grid = (unsigned)((n + 63) / 64);
     const auto kernel = N <= 16   ? localized_mfma_kernel<1>
                         : N <= 32 ? localized_mfma_kernel<2>
@@ -620,7 +651,8 @@ void ensemble_analysis(Ensemble &ens, double *T, int n_params, double *params,
   bool finite = true;
   for (double v : S) finite = finite && std::isfinite(v);
   for (double v : Ek) finite = finite && std::isfinite(v);
-  launch_localized(finite, T, N, n, d_S, d_E, d_oc, m, fn, cutoff, geo, s);
+  launch_localized(finite && localized_mfma_pays(N, n, m, cutoff, geo), T, N, n,
+                   d_S, d_E, d_oc, m, fn, cutoff, geo, s);
   ADM_HIP_DA(hipGetLastError());
 }
 

@@ -67,3 +67,53 @@ def test_localized_update_not_finite_reaches_all():
     assert far.any()
     np.testing.assert_allclose(got[:, far], X[:, far], rtol=1e-14)
     assert not np.isfinite(got[:, obs]).any()
+
+
+def direct_update(X, xyz, obs, y, R, noise, fn, cutoff):
+    """x_j + rho o (A^T S) (rho o (S^T S) / (N-1) + R)^-1 d_j / (N-1)."""
+    def rho(d):
+        if fn == "step_function":
+            return (d <= cutoff).astype(float)
+        q = 2.0 * d / cutoff
+        near = ((((-0.25 * q + 0.5) * q + 0.625) * q - 5.0 / 3.0) * q * q
+                + 1.0)
+        s = np.maximum(q, 1.0)
+        far = ((((s / 12.0 - 0.5) * s + 0.625) * s + 5.0 / 3.0) * s - 5.0) \
+            * s + 4.0 - 2.0 / (3.0 * s)
+        return np.where(q < 1.0, near, np.where(q < 2.0, far, 0.0))
+    N = len(X)
+    A = X - X.mean(0)
+    S, xo = A[:, obs], xyz[obs]
+    dist = np.linalg.norm(xo[:, None] - xo, axis=2)
+    E = np.linalg.solve(rho(dist) * (S.T @ S) / (N - 1) + R,
+                        (noise + y - X[:, obs]).T)
+    out = X.copy()
+    for k in range(len(obs)):
+        w = rho(np.linalg.norm(xyz - xo[k], axis=1)) * (S[:, k] @ A) / (N - 1)
+        out += np.outer(E[k], w)
+    return out
+
+
+@pytest.mark.parametrize("fn", ["step_function", "gaspari_cohn"])
+@pytest.mark.parametrize("N,m,cutoff", [
+    (2, 1, 0.2e-3), (2, 17, 3e-3), (5, 3, 1e-3), (8, 64, 3e-3),
+    (16, 2, 0.5e-3), (16, 40, 3e-3), (17, 1, 1e-3), (17, 20, 1e-3),
+    (32, 1, 0.2e-3), (32, 33, 1e-3), (33, 1, 1e-3)])
+def test_localized_update_large(N, m, cutoff, fn):
+    """A mesh on which some sizes take the lane-per-node kernel and some the
+    matrix tiles."""
+    from adamantine_amd.ensemble import EnsembleDevice, Member
+    from adamantine_amd.workloads import plain_large
+    base = plain_large(n_cells=(61, 32, 17))
+    ens = EnsembleDevice(base, [Member() for _ in range(N)])
+    rng = np.random.RandomState(100 * N + m)
+    X = 1000.0 + rng.normal(scale=30.0, size=(N, ens.n_dofs))
+    obs = np.sort(rng.permutation(ens.n_dofs)[:m]).astype(np.int64)
+    y = 1000.0 + rng.normal(scale=5.0, size=m)
+    R, noise = np.diag(rng.uniform(1.0, 4.0, m)), rng.normal(0.0, 1.5, (N, m))
+    got = update(ens, base, fn, cutoff, X, obs, y, R, noise)
+    want = direct_update(X, base.node_coordinates(), obs, y, R, noise, fn,
+                         cutoff)
+    scale = np.abs(want - X).max()
+    assert scale > 0.1
+    assert np.abs(got - want).max() <= 1e-10 * scale + 1e-12 * 1000
