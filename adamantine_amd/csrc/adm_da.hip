@@ -560,13 +560,7 @@ void ensemble_analysis(Ensemble &ens, double *T, int n_params, double *params,
   if (fn == ADM_LOCALIZATION_GASPARI_COHN &&
       !(gaspari_cohn(2.0 * diag / cutoff) == 1.0))
     localized = true;
-  bool r_diag = true;
-  for (int a = 0; a < m && r_diag; ++a)
-    for (int b = 0; b < m; ++b)
-      if (a != b && R[(size_t)a * m + b] != 0.0) {
-        r_diag = false;
-        break;
-      }
+  const bool r_diag = is_diagonal(m, R);
   const double nm1 = N - 1.0;
   // W0 = S E / (N-1) (N x N, [l][j]); E = C^{-1} D^T (m x N, column j of D)
   std::vector<double> W0, E;  // E row-major [m][N]

@@ -112,6 +112,21 @@ static bool has_avx2() {
 static bool has_avx2() { return false; }
 #endif
 
+// Whether every off-diagonal entry of an m x m row-major matrix is zero (a
+// value that is not a number is not). Without a branch in a row: with one per
+// entry an analysis of 2 members and 400 observations took 115 us, 139 once
+// the code around it had changed, and takes 85 so.
+static __attribute__((noinline)) bool is_diagonal(int m, const double *R) {
+  for (int a = 0; a < m; ++a) {
+    const double *row = R + (size_t)a * m;
+    int other = 0;
+    for (int b = 0; b < a; ++b) other |= row[b] != 0.0;
+    for (int b = a + 1; b < m; ++b) other |= row[b] != 0.0;
+    if (other) return false;
+  }
+  return true;
+}
+
 #undef ADM_BODY
 
 }  // namespace adm

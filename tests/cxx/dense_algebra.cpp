@@ -15,4 +15,8 @@ void gram(int body, int m, int p, const double *X, int q, const double *Y,
   (body ? adm::gram_avx2 : adm::gram_plain)(m, p, X, q, Y, C);
 }
 
+int is_diagonal(int m, const double *R) {
+  return adm::is_diagonal(m, R) ? 1 : 0;
+}
+
 }

@@ -133,3 +133,22 @@ def test_bodies_agree(lib, seed):
     for body in (0, 1):
         lib.gram(body, m, m, ptr(A), 19, ptr(B), ptr(C[body]))
     np.testing.assert_array_equal(C[0], C[1])
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 8, 33])
+def test_is_diagonal(lib, m):
+    R = np.diag(np.arange(m, dtype=float))  # a zero on the diagonal too
+    assert lib.is_diagonal(m, ptr(R)) == 1
+    R[0, 0] = np.nan
+    assert lib.is_diagonal(m, ptr(R)) == 1
+    for a, b in ((0, m - 1), (m - 1, 0), (m // 2, 0), (m - 1, m - 2)):
+        for v in (1e-300, -1.0, np.nan, np.inf):
+            if a == b or b < 0:
+                continue
+            Q = R.copy()
+            Q[a, b] = v
+            assert lib.is_diagonal(m, ptr(Q)) == 0, (a, b, v)
+        if a != b and b >= 0:
+            Q = R.copy()
+            Q[a, b] = -0.0
+            assert lib.is_diagonal(m, ptr(Q)) == 1
